@@ -1,13 +1,15 @@
 // lx_matmul.hip -- MatMul on gfx950 (Tensor<T>.MatMul, TensorOps.cs:504-806,
 // via CPUExecutionProvider.MatMul, CPUExecutionProvider.cs:359-378).
 //
-// float : v_mfma_f32_32x32x2f32 (fp32 products, fp32 accumulation -- the
-//         reference's float32 arithmetic, summed in a different order, the
-//         same order in both kernels).  K a multiple of 64 with aligned
-//         operands: a ring of LDS stages filled by direct-to-LDS loads two or
-//         three K steps ahead (k_matmul_f32_dl); otherwise double-buffered LDS
-//         fed from registers one K step ahead (k_matmul_f32).  Block tiles
-//         from 64x64 to 128x128 chosen per shape, K step 16, four waves.
+// float : K ranges of 256 and more (N above 32): every operand in three bf16
+//         parts on v_mfma_f32_32x32x16_bf16 (k_matmul_f32_b3), closer to 64
+//         bits than float32 products and 2.2 times the rate.  Shorter ones:
+//         v_mfma_f32_32x32x2f32 (fp32 products, fp32 accumulation), summed in
+//         one order by two kernels: K a multiple of 64 with aligned operands
+//         through a ring of LDS stages filled by direct-to-LDS loads
+//         (k_matmul_f32_dl), otherwise double-buffered LDS fed from registers
+//         one K step ahead (k_matmul_f32).  Block tiles from 64x64 to 128x128
+//         chosen per shape, K step 16, four waves.
 // double: v_mfma_f64_16x16x4f64, 64x64 block tile, four waves of 32x32.
 // int32 : exact two's-complement multiply-add on the VALU (no int32 MFMA),
 //         16x16 LDS tiles.
@@ -606,10 +608,463 @@ static void launch_f32_dl(const float *a, const float *b, float *c, const MatMul
     else hipLaunchKernelGGL((k_matmul_f32_dl<BM, BN, WM, WN, 4, WMIN, WMAX, false>), g, blk, 0, s, a, b, c, p);
 }
 
+// ---------------------------------------------------------------------------
+// float, K ranges of 256 or more: every operand in three bf16 parts on the bf16 matrix unit
+// ---------------------------------------------------------------------------
+// x = p1 + p2 + p3 with p1 = bf16(x), p2 = bf16(x - p1), p3 = bf16(x - p1 - p2): three 8-bit significands hold all 24
+// bits of a float32, so the parts of a value of 2^-109 or more are exact.  A product is the six part products of
+// weight 2^-16 or more,
+//   a3 b1 + a1 b3 + a2 b2 + a2 b1 + a1 b2 + a1 b1
+// (the three left out weigh 2^-25 |a b| at most), each exact in the MFMA and accumulated in float32: per step of 16
+// six v_mfma_f32_32x32x16_bf16 of 32 cycles, where v_mfma_f32_32x32x2f32 takes eight of 64.  Against 64 bits, normal
+// data, the relative error is below the fp32 MFMA's at every K: 1.6e-7 against 2.0e-7 (K 128), 2.9e-7 / 3.5e-7 (384),
+// 4.2e-7 / 5.0e-7 (768), 8.6e-7 / 1.0e-6 (3072), the small part products first as above (largest first: 1.8e-7 at
+// 128).  Shorter ranges stay on the fp32 MFMA: they are bound by launches and loads ([667,384]x[384,384] in ranges of
+// 128 ran slower in parts).  The choice is by the length of the K range alone, so that a product is the same bits in every tile, fused or not, folded or not.
+//
+// What the parts cannot hold goes to the fp32 MFMA, element by element: values that are not finite (or round to an
+// infinite bf16) make the result not finite, and parts below 2^-133 are lost, which a result smaller than 2^-90 of
+// its row's and column's largest operand can show.  Each thread keeps the largest magnitude it loaded of its row and
+// column; a wave holding such a result runs that 32x32 tile again from global memory (f32_tile) and takes those
+// elements from it.  (A row or column of zeros needs no second run: its results are zero.)
+//
+// Bound: the matrix unit (register-only, 340 TFLOP/s of float32 products at the clock it holds), then the issue slots
+// of the splitting (11 VALU instructions per pair of elements) and of LDS, so each element is split once per block,
+// on its way from global memory to LDS, and the splitting, the LDS accesses and the loads are dealt out between the
+// MFMAs one by one (in runs they stalled the wave's MFMAs: [4096,3072]x[3072,768] 208 us with the phases one after
+// another, 130 with fragments a step ahead, 112 dealt out evenly with eight waves).  Stage layout: per 16-k sub-step
+// and part, [k half][row] chunks of eight bf16, the halves 64 bytes apart modulo 256: the 16-byte fragment reads and
+// the writes are free of bank conflicts.  Two stages: step t multiplies the fragments read during step t - 1, reads
+// those of step t + 1, writes the parts of step t + 2 into the stage they left and loads step t + 4.
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t bf16_pair(float x0, float x1) {
+    const v2f x = {x0, x1};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, v2bf));
+}
+
+// one 32x32 tile of the product over k in [k0, k1), rows row0.. and columns col0.. (clamped to M, N), straight from
+// global memory on the fp32 MFMA in the fp32 kernels' order
+template <bool BT>
+__device__ __noinline__ v16f f32_tile(const float *A, const float *B, int M, int N, int64_t lda, int64_t ldb, int row0,
+                                      int col0, int k0, int k1, int l) {
+    const int h = l / 32;
+    const float *ar = A + (int64_t)min(row0 + l % 32, M - 1) * lda;
+    const int64_t col = min(col0 + l % 32, N - 1);
+    v16f acc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.f;
+    for (int k = k0; k < k1; k += 16) {
+        float a[8], b[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int kk = k + 8 * h + j;
+            a[j] = kk < k1 ? ar[kk] : 0.f;
+            b[j] = kk < k1 ? (BT ? B[col * ldb + kk] : B[(int64_t)kk * ldb + col]) : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(b[j], a[j], acc, 0, 0, 0);
+    }
+    return acc;
+}
+
+// BM x BN tile, WM x WN multiplying waves, KS sub-steps of 16 per step, WE waves per SIMD.  PW: loading waves that
+// load and split for them (0: every wave does both).  A block alone on its CU is bound by its waves' issue slots, not
+// by the matrix unit: eight loading waves beside the four of a 64x64 tile take [788,3072]x[3072,768] (156 tiles) from
+// 57 to 44 us; with several blocks per CU, or 128x128 tiles, both forms run alike or the joint one faster ([4096,768]x
+// [768,3072] 107 against 120 us).  VEC: 16-byte loads along K (the rows
+// of A, and of B by columns, 16-byte aligned).  TAIL: the K range is no whole number of step pairs (past it the loads
+// clamp to the last step's and their elements are zeroed).  vc: 16-byte epilogue.  SPLIT as in k_matmul_f32_dl.
+template <int BM, int BN, int WM, int WN, int PW, int KS, int WE, bool VEC, bool TAIL, bool BT, bool GELU,
+          bool SPLIT = false>
+__global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_per_eu(WE, WE))) void k_matmul_f32_b3(
+    const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, MatMulArgs p, int vc) {
+    constexpr int NW = WM * WN, NTHR = (PW ? PW : NW) * 64, KB = 16 * KS;  // NTHR: the threads that load and split
+    constexpr int MT = BM / WM / 32, NT = BN / WN / 32;
+    static_assert(MT * WM * 32 == BM && NT * WN * 32 == BN, "waves of whole 32x32 tiles");
+    constexpr int AH = BM * 16 + 64, BH = BN * 16 + 64;         // bytes of a k half of one part (64: the bank offset)
+    constexpr int AP = 2 * AH, BP = 2 * BH, SUB = 3 * (AP + BP), STAGE = SUB * KS;
+    constexpr int CA = BM * KB / NTHR >= 8 ? 8 : 4, NA = BM * KB / CA / NTHR;  // floats per chunk, chunks per thread
+    constexpr int CB = BN * KB / NTHR >= 8 ? 8 : 4, NB = BN * KB / CB / NTHR;
+    static_assert(NA * CA * NTHR == BM * KB && NB * CB * NTHR == BN * KB, "whole chunks");
+    __shared__ __attribute__((aligned(1024))) char sm[2][STAGE];
+    __shared__ uint32_t amax[BM], bmax[BN];  // bits of the largest magnitude of each row and column
+    __shared__ ExpTable tab;
+    if constexpr (GELU) exp_table_fill(tab);
+    const int M = p.m, N = p.n;
+    const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = (int)threadIdx.x - (PW ? NW * 64 : 0);  // index among the threads that load and split
+    const int row0 = blockIdx.y * BM, col0 = blockIdx.x * BN;
+    const int zb = SPLIT ? (int)blockIdx.z / p.split : (int)blockIdx.z;
+    const int kr = SPLIT ? p.k / p.split : p.k;                       // length of the K range
+    const int kbeg = SPLIT ? ((int)blockIdx.z - zb * p.split) * kr : 0;
+    const int nk = 2 * ((kr + 2 * KB - 1) / (2 * KB));                // steps, in pairs
+    int64_t ao, bo, co;
+    batch_offsets(p.batch_base + zb, p, &ao, &bo, &co);
+    for (int i = threadIdx.x; i < BM; i += blockDim.x) amax[i] = 0;
+    for (int i = threadIdx.x; i < BN; i += blockDim.x) bmax[i] = 0;
+
+    // this thread's chunks: A chunk h is CA floats along K of one row (byte offset aoff, LDS offset ad); B chunk h is
+    // CB k of one column (b by columns: as A's)
+    int aoff[NA], ak[NA], ad[NA], ar[NA], boff[NB], bk[NB], bd[NB], bc[NB];
+#pragma unroll
+    for (int h = 0; h < NA; h++) {
+        const int q = t + NTHR * h, r = q / (KB / CA), c = q % (KB / CA) * CA;
+        ar[h] = r;
+        ak[h] = c;
+        aoff[h] = (int)(((int64_t)min(r, M - 1 - row0) * p.lda + c) * 4);
+        ad[h] = c / 16 * SUB + c % 16 / 8 * AH + r * 16 + c % 8 * 2;
+    }
+#pragma unroll
+    for (int h = 0; h < NB; h++) {
+        const int q = t + NTHR * h;
+        const int c = BT ? q / (KB / CB) : q % BN;
+        int k = BT ? q % (KB / CB) * CB : q / BN * CB;
+        if constexpr (!BT && BN >= 64) k = __builtin_amdgcn_readfirstlane(k);
+        bc[h] = c;
+        bk[h] = k;
+        const int cc = min(c, N - 1 - col0);
+        boff[h] = (int)((BT ? (int64_t)cc * p.ldb + k : (int64_t)k * p.ldb + cc) * 4);
+        bd[h] = k / 16 * SUB + 3 * AP + k % 16 / 8 * BH + c * 16 + k % 8 * 2;
+    }
+    const char *Ab = (const char *)(A + ao + (int64_t)row0 * p.lda + kbeg);
+    const char *Bb = (const char *)(B + bo + (BT ? (int64_t)col0 * p.ldb + kbeg : (int64_t)kbeg * p.ldb + col0));
+    const int64_t bstep = BT ? (int64_t)KB * 4 : (int64_t)KB * p.ldb * 4;  // bytes per step
+    const int ldb4 = BT ? 4 : (int)p.ldb * 4;                              // bytes between a B chunk's elements
+    // buffer loads: a step's base in scalar registers, one 32-bit offset per lane (all in range: the host bounds the
+    // strides, rows, columns and k are clamped)
+    auto rsrc = [](const char *b) { return __builtin_amdgcn_make_buffer_rsrc((void *)b, 0, 0x7fffffff, 0x00027000); };
+    // k index within the range of element e of a chunk at k c of step kt, clamped in the tail: offset back in bytes
+    struct Set {
+        float a[NA][CA], b[NB][CB];
+    };
+    // loads elements e .. e + n - 1 (n = 4 with VEC) of chunk h of step kt
+    auto load_a = [&](Set &s, auto hc, auto ec, int kt) {
+        constexpr int h = decltype(hc)::value, e = decltype(ec)::value;
+        const auto rs = rsrc(Ab + (int64_t)kt * (KB * 4));
+        const int lim = TAIL ? kr - kt * KB : 0;  // k left in the range at this step (may be below 1)
+        if constexpr (VEC) {
+            int o = aoff[h] + e * 4;
+            if constexpr (TAIL) o -= max(0, ak[h] + e + 4 - lim) * 4;
+            const v4f v = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rs, o, 0, 0));
+#pragma unroll
+            for (int z = 0; z < 4; z++) s.a[h][e + z] = v[z];
+        } else {
+#pragma unroll
+            for (int z = 0; z < 4; z++) {
+                const int o = aoff[h] + (e + z) * 4 - max(0, ak[h] + e + z + 1 - lim) * 4;
+                s.a[h][e + z] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, o, 0, 0));
+            }
+        }
+    };
+    auto load_b = [&](Set &s, auto hc, auto ec, int kt) {  // by columns: elements e .. e + 3; else e and e + 1
+        constexpr int h = decltype(hc)::value, e = decltype(ec)::value;
+        const auto rs = rsrc(Bb + kt * bstep);
+        const int lim = TAIL ? kr - kt * KB : 0;
+        if constexpr (BT && VEC) {
+            int o = boff[h] + e * 4;
+            if constexpr (TAIL) o -= max(0, bk[h] + e + 4 - lim) * 4;
+            const v4f v = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rs, o, 0, 0));
+#pragma unroll
+            for (int z = 0; z < 4; z++) s.b[h][e + z] = v[z];
+        } else {
+#pragma unroll
+            for (int z = 0; z < (BT ? 4 : 2); z++) {
+                int so = (e + z) * ldb4;
+                int o = boff[h];
+                if constexpr (TAIL) {
+                    const int back = max(0, bk[h] + e + z + 1 - lim);
+                    o += so - back * ldb4;
+                    so = 0;
+                }
+                s.b[h][e + z] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, o, so, 0));
+            }
+        }
+    };
+    auto load_all = [&](Set &s, int kt) {
+        static_for<0, NA>([&](auto h) {
+            static_for<0, CA / 4>([&](auto e) { load_a(s, h, std::integral_constant<int, 4 * decltype(e)::value>(), kt); });
+        });
+        static_for<0, NB>([&](auto h) {
+            constexpr int n = BT ? 4 : 2;
+            static_for<0, CB / n>([&](auto e) { load_b(s, h, std::integral_constant<int, n * decltype(e)::value>(), kt); });
+        });
+    };
+
+    // splitting: the pairs of a thread's chunks in units of four, twelve segments per unit, in each segment one
+    // instruction (or two) per pair, so that neighbouring instructions are independent
+    constexpr int PA = NA * CA / 2, PB = NB * CB / 2, PT = PA + PB, U = (PT + 3) / 4, SEGS = 12 * U;
+    float mxa[NA], mxb[NB];
+#pragma unroll
+    for (int h = 0; h < NA; h++) mxa[h] = 0.f;
+#pragma unroll
+    for (int h = 0; h < NB; h++) mxb[h] = 0.f;
+    float res[8];
+    uint32_t hi[8], pk[3][PT];
+    // segment ic of the split of step kt's elements in s into stage ws; then loads step kl into s
+    auto segment = [&](auto ic, Set &s, int kt, char *ws, int kl) {
+        constexpr int i = decltype(ic)::value, un = i / 12, sg = i % 12, np = PT - 4 * un < 4 ? PT - 4 * un : 4;
+        static_for<0, np>([&](auto qc) {
+            constexpr int q = decltype(qc)::value, pr = 4 * un + q;
+            constexpr bool isA = pr < PA;
+            constexpr int CN = isA ? CA : CB, qq = isA ? pr : pr - PA, h = qq / (CN / 2), e = qq % (CN / 2) * 2;
+            float *x;
+            if constexpr (isA) x = &s.a[h][e];
+            else x = &s.b[h][e];
+            if constexpr (sg == 0) {
+                if constexpr (TAIL) {
+                    const int k = (isA ? ak[isA ? h : 0] : bk[isA ? 0 : h]) + e, lim = kr - kt * KB;
+                    x[0] = k < lim ? x[0] : 0.f;
+                    x[1] = k + 1 < lim ? x[1] : 0.f;
+                }
+                pk[0][pr] = bf16_pair(x[0], x[1]);
+            }
+            if constexpr (sg == 1 || sg == 6) hi[2 * q] = pk[sg / 6][pr] << 16;
+            if constexpr (sg == 2 || sg == 7) hi[2 * q + 1] = pk[sg / 6][pr] & 0xffff0000u;
+            if constexpr (sg == 3) res[2 * q] = x[0] - __builtin_bit_cast(float, hi[2 * q]);
+            if constexpr (sg == 4) res[2 * q + 1] = x[1] - __builtin_bit_cast(float, hi[2 * q + 1]);
+            if constexpr (sg == 5) {
+                pk[1][pr] = bf16_pair(res[2 * q], res[2 * q + 1]);
+                float &m = isA ? mxa[isA ? h : 0] : mxb[isA ? 0 : h];
+                m = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), m);
+            }
+            if constexpr (sg == 8) res[2 * q] -= __builtin_bit_cast(float, hi[2 * q]);
+            if constexpr (sg == 9) res[2 * q + 1] -= __builtin_bit_cast(float, hi[2 * q + 1]);
+            if constexpr (sg == 10) pk[2][pr] = bf16_pair(res[2 * q], res[2 * q + 1]);
+            if constexpr (e + 2 == CN && (sg == 1 || sg == 6 || sg == 11)) {  // part sg / 5 of the chunk is complete
+                constexpr int z = sg / 5, p0 = pr + 1 - CN / 2;
+                char *d = ws + (isA ? ad[isA ? h : 0] : bd[isA ? 0 : h]) + z * (isA ? AP : BP);
+                if constexpr (CN == 8) *(v4u *)d = v4u{pk[z][p0], pk[z][p0 + 1], pk[z][p0 + 2], pk[z][p0 + 3]};
+                else *(v2u *)d = v2u{pk[z][p0], pk[z][p0 + 1]};
+            }
+            // the elements are in parts: reload them
+            if constexpr (isA) {
+                if constexpr (e % 4 == 2 && sg == 7 + q / 2)
+                    load_a(s, std::integral_constant<int, h>(), std::integral_constant<int, e - 2>(), kl);
+            } else if constexpr (BT) {
+                if constexpr (e % 4 == 2 && sg == 7 + q / 2)
+                    load_b(s, std::integral_constant<int, h>(), std::integral_constant<int, e - 2>(), kl);
+            } else if constexpr (sg == 6 + q) {
+                load_b(s, std::integral_constant<int, h>(), std::integral_constant<int, e>(), kl);
+            }
+        });
+    };
+
+    // the largest operand of each row and column
+    auto store_max = [&]() {
+#pragma unroll
+        for (int h = 0; h < NA; h++) atomicMax(&amax[ar[h]], __builtin_bit_cast(uint32_t, mxa[h]));
+#pragma unroll
+        for (int h = 0; h < NB; h++) atomicMax(&bmax[bc[h]], __builtin_bit_cast(uint32_t, mxb[h]));
+    };
+    // parts of steps 0 and 1 into their stages, steps 2 and 3 loading
+    Set s0, s1;
+    auto prologue = [&]() {
+        load_all(s0, 0);
+        load_all(s1, 1);
+        static_for<0, SEGS>([&](auto c) { segment(c, s0, 0, sm[0], min(2, nk - 1)); });
+        static_for<0, SEGS>([&](auto c) { segment(c, s1, 1, sm[1], min(3, nk - 1)); });
+        wait_vmcnt_barrier<63>();
+    };
+    if constexpr (PW > 0) {
+        if (w >= NW) {  // a loading wave: step by step with the barriers of the multiplying ones
+            prologue();
+            wait_vmcnt_barrier<63>();
+            auto produce = [&](int kt, Set &s) {
+                static_for<0, SEGS>([&](auto c) { segment(c, s, kt + 2, sm[kt & 1], min(kt + 4, nk - 1)); });
+                wait_vmcnt_barrier<63>();
+            };
+            for (int kt = 0; kt < nk; kt += 2) {
+                produce(kt, s0);
+                produce(kt + 1, s1);
+            }
+            store_max();
+            __syncthreads();
+            return;
+        }
+    }
+
+    const int wr = (w / WN) * MT * 32, wc = (w % WN) * NT * 32;
+    const int fa = (wr + (l & 31)) * 16 + AH * (l >> 5), fb = 3 * AP + (wc + (l & 31)) * 16 + BH * (l >> 5);
+    struct Frag {
+        v8bf a[KS][3][MT], b[KS][3][NT];
+    };
+    constexpr int RF = 3 * (MT + NT), R = RF * KS;  // fragment reads per step, in the order of their first use
+    auto read_frag = [&](auto ic, const char *rs, Frag &f) {
+        constexpr int i = decltype(ic)::value, u = i / RF, o = i % RF / (MT + NT), z = i % RF % (MT + NT);
+        constexpr int pa = o == 0 ? 2 : o == 1 ? 0 : 1, pb = o == 0 ? 0 : o == 1 ? 2 : 1;
+        if constexpr (z < MT) f.a[u][pa][z] = *(const v8bf *)(rs + u * SUB + pa * AP + fa + z * 512);
+        else f.b[u][pb][z - MT] = *(const v8bf *)(rs + u * SUB + pb * BP + fb + (z - MT) * 512);
+    };
+    v16f acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+    constexpr int G = 6 * MT * NT * KS, GD = G * 5 / 6;  // MFMAs per step; the other work follows the first GD of them
+    auto step = [&](int kt, Set &s, const Frag &cur, Frag &nxt) {
+        const char *rs = sm[(kt + 1) & 1];
+        char *ws = sm[kt & 1];
+        const int kl = min(kt + 4, nk - 1);
+        static_for<0, G>([&](auto gc) {
+            constexpr int g = decltype(gc)::value, u = g / (6 * MT * NT), o = g % (6 * MT * NT), pr = o / (MT * NT);
+            constexpr int i = o % (MT * NT) / NT, j = o % NT;
+            constexpr int pa = pr == 0 ? 2 : pr == 1 || pr >= 4 ? 0 : 1, pb = pr == 1 ? 2 : pr == 2 || pr == 4 ? 1 : 0;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.b[u][pb][j], cur.a[u][pa][i], acc[i][j], 0, 0, 0);
+            static_for<(g < GD ? g * R / GD : R), (g < GD ? (g + 1) * R / GD : R)>([&](auto c) { read_frag(c, rs, nxt); });
+            if constexpr (PW == 0)
+                static_for<(g < GD ? g * SEGS / GD : SEGS), (g < GD ? (g + 1) * SEGS / GD : SEGS)>(
+                    [&](auto c) { segment(c, s, kt + 2, ws, kl); });
+            sched_fence();
+        });
+        // every wave's LDS reads and writes are done before the stages change roles (the loads stay outstanding)
+        wait_vmcnt_barrier<63>();
+    };
+    Frag f0, f1;
+    if constexpr (PW > 0) wait_vmcnt_barrier<63>();
+    else prologue();
+    static_for<0, R>([&](auto c) { read_frag(c, sm[0], f0); });
+    wait_vmcnt_barrier<63>();  // stage 0 is read before step 0 writes it
+    for (int kt = 0; kt < nk; kt += 2) {
+        step(kt, s0, f0, f1);
+        step(kt + 1, s1, f1, f0);
+    }
+
+    // the results the parts cannot hold
+    if constexpr (PW == 0) store_max();
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+        const float ra = __builtin_bit_cast(float, amax[wr + 32 * i + (l & 31)]);
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            uint32_t again = 0;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const float cb = __builtin_bit_cast(float, bmax[wc + 32 * j + 8 * (r / 4) + 4 * (l / 32) + r % 4]);
+                const float v = fabsf(acc[i][j][r]);
+                const bool ok = v >= fmaxf(ra, cb) * 0x1p-90f && v < __builtin_inff();
+                again |= (ok || ra == 0.f || cb == 0.f) ? 0u : 1u << r;
+            }
+            // (a zero row times an infinite or NaN column is not finite)
+#pragma unroll
+            for (int r = 0; r < 16; r++) again |= fabsf(acc[i][j][r]) < __builtin_inff() ? 0u : 1u << r;
+            if (__any(again != 0)) {
+                const v16f x = f32_tile<BT>(A + ao, B + bo, M, N, p.lda, p.ldb, row0 + wr + 32 * i, col0 + wc + 32 * j,
+                                            kbeg, kbeg + kr, l);
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    if (again >> r & 1) acc[i][j][r] = x[r];
+            }
+        }
+    }
+    if constexpr (SPLIT)
+        mm_store_part<MT, NT>(acc, p.part + ((int64_t)(blockIdx.z - zb * p.split) * p.batch + zb) * M * N, M, N,
+                              row0 + wr, col0 + wc, l);
+    else if (vc)
+        mm_epilogue<MT, NT, true, GELU>(acc, C, p, co, row0 + wr, col0 + wc, l, tab);
+    else
+        mm_epilogue<MT, NT, false, GELU>(acc, C, p, co, row0 + wr, col0 + wc, l, tab);
+}
+
+constexpr int kB3MinK = 256;
+// Whether a K range of kr goes to k_matmul_f32_b3: kB3MinK or more, N above 32 (a context product of 32-wide heads is
+// bound by its loads: [96,512,512]x[96,512,32] 24 us on the fp32 MFMA, 26 in parts), and strides whose offsets within
+// a tile and a step stay below 2^31 bytes (rows of up to 8 MB; longer ones keep the fp32 MFMA).
+static bool f32_b3(const MatMulArgs &p, int kr) {
+    const int64_t lim = (int64_t)1 << 21;
+    return kr >= kB3MinK && p.n > 32 && p.lda <= lim && p.ldb <= lim && p.k <= (1 << 24);
+}
+
+// The block tile: the least estimated time.  A tile's step of 16 k takes `lone` us when its block has a CU to itself
+// and `full` us per block with r of them on a CU, measured over [4096, 384..3072] x [.., 384..3072], [788, ..] and
+// 2048^3: rounds of r blocks, then the rest.  64x64 with loading waves (12 waves: one block per CU) only up to 256
+// tiles.
+static int b3_tile(const MatMulArgs &p, bool only_general) {
+    struct B3Tile {
+        int bm, bn, r;
+        double lone, full;
+    };
+    static const B3Tile cand[] = {{128, 128, 2, 0.57, 0.72}, {128, 64, 2, 0.40, 0.50}, {64, 64, 3, 0.25, 0.25},
+                                  {64, 64, 1, 0.215, 0.39}};
+    int best = 0;
+    double cost = 0;
+    for (int i = 0; i < 4; i++) {
+        if (only_general && (i == 1 || i == 3)) continue;
+        const B3Tile &c = cand[i];
+        const int64_t tiles = (int64_t)((p.m + c.bm - 1) / c.bm) * ((p.n + c.bn - 1) / c.bn) * p.batch;
+        const int64_t per_cu = (tiles + 255) / 256, rounds = per_cu / c.r, rest = per_cu - rounds * c.r;
+        const double t = per_cu == 1 ? c.lone : rounds * c.r * c.full + (rest > 1 ? rest * c.full : rest * c.lone);
+        if (i == 0 || t < cost) {
+            best = i;
+            cost = t;
+        }
+    }
+    return best;
+}
+
+template <int BM, int BN, int WM, int WN, int PW, int KS, int WE, bool VEC, bool TAIL, bool BT>
+static void b3_launch(const float *a, const float *b, float *c, const MatMulArgs &p, bool vc, hipStream_t s) {
+    const dim3 g((p.n + BN - 1) / BN, (p.m + BM - 1) / BM, (unsigned)p.batch), blk((WM * WN + PW) * 64);
+    if constexpr (!BT) {
+        if (p.gelu) {
+            hipLaunchKernelGGL((k_matmul_f32_b3<BM, BN, WM, WN, PW, KS, WE, VEC, TAIL, false, true>), g, blk, 0, s, a, b, c, p, (int)vc);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_matmul_f32_b3<BM, BN, WM, WN, PW, KS, WE, VEC, TAIL, BT, false>), g, blk, 0, s, a, b, c, p, (int)vc);
+}
+
+// vec: f32_vec (the epilogue's 16-byte accesses)
+static void launch_f32_b3(const float *a, const float *b, float *c, const MatMulArgs &p, bool vec, hipStream_t s) {
+    // 16-byte loads along K: A's rows (and B's columns, by columns) aligned, K a multiple of 4
+    bool va = p.k % 4 == 0 && p.lda % 4 == 0 && (uintptr_t)a % 16 == 0 &&
+              (!p.bt || (p.ldb % 4 == 0 && (uintptr_t)b % 16 == 0));
+    for (int d = 0; d < p.nbatch; d++) va = va && p.a_bstr[d] % 4 == 0 && (!p.bt || p.b_bstr[d] % 4 == 0);
+    const bool whole = va && p.k % 64 == 0;  // whole step pairs of every tile
+    const int tile = b3_tile(p, p.bt || !whole);
+    if (p.bt) {
+        if (whole && tile == 0) b3_launch<128, 128, 2, 4, 0, 1, 4, true, false, true>(a, b, c, p, vec, s);
+        else if (whole) b3_launch<64, 64, 2, 2, 0, 2, 3, true, false, true>(a, b, c, p, vec, s);
+        else b3_launch<64, 64, 2, 2, 0, 2, 2, false, true, true>(a, b, c, p, vec, s);
+        return;
+    }
+    if (!va) {  // unaligned rows: scalar loads
+        if (tile == 0) b3_launch<128, 128, 2, 4, 0, 1, 4, false, true, false>(a, b, c, p, vec, s);
+        else b3_launch<64, 64, 2, 2, 0, 2, 2, false, true, false>(a, b, c, p, vec, s);
+        return;
+    }
+    if (!whole) {
+        if (tile == 0) b3_launch<128, 128, 2, 4, 0, 1, 4, true, true, false>(a, b, c, p, vec, s);
+        else b3_launch<64, 64, 2, 2, 0, 2, 2, true, true, false>(a, b, c, p, vec, s);
+        return;
+    }
+    switch (tile) {
+    case 0: b3_launch<128, 128, 2, 4, 0, 1, 4, true, false, false>(a, b, c, p, vec, s); break;
+    case 1: b3_launch<128, 64, 4, 2, 0, 2, 2, true, false, false>(a, b, c, p, vec, s); break;
+    case 2: b3_launch<64, 64, 2, 2, 0, 2, 3, true, false, false>(a, b, c, p, vec, s); break;
+    default: b3_launch<64, 64, 2, 2, 8, 2, 3, true, false, false>(a, b, c, p, vec, s); break;
+    }
+}
+
+// the K ranges of a split product into p.part: 64x64 tiles, at most one per CU
+static void launch_f32_parts(const float *a, const float *b, float *c, const MatMulArgs &p, hipStream_t s) {
+    const dim3 g((p.n + 63) / 64, (p.m + 63) / 64, (unsigned)(p.batch * p.split));
+    if (f32_b3(p, p.k / p.split))
+        hipLaunchKernelGGL((k_matmul_f32_b3<64, 64, 2, 2, 8, 2, 3, true, false, false, false, true>), g, dim3(768), 0, s, a, b, c, p, 1);
+    else
+        hipLaunchKernelGGL((k_matmul_f32_dl<64, 64, 2, 2, 4, 3, 8, false, true>), g, dim3(256), 0, s, a, b, c, p);
+}
+
 // Split K (p.split ranges, p.part holding the partials): 64x64 tiles, then the ordered sum with the epilogue.
 static void launch_f32_split(const float *a, const float *b, float *c, const MatMulArgs &p, hipStream_t s) {
-    dim3 g((p.n + 63) / 64, (p.m + 63) / 64, (unsigned)(p.batch * p.split));
-    hipLaunchKernelGGL((k_matmul_f32_dl<64, 64, 2, 2, 4, 3, 8, false, true>), g, dim3(256), 0, s, a, b, c, p);
+    launch_f32_parts(a, b, c, p, s);
     const int64_t nq = (int64_t)p.m * p.n / 4 * p.batch;
     const dim3 gs((unsigned)((nq + 255) / 256));
     if (p.gelu) hipLaunchKernelGGL(k_matmul_split_sum<true>, gs, dim3(256), 0, s, c, p);
@@ -868,9 +1323,7 @@ hipError_t launch_matmul_ln(const void *a, const void *b, void *y, const MatMulA
     if (!matmul_ln_fusable(kFloat, a, b, y, p0) || !p0.part) return hipErrorInvalidValue;
     MatMulArgs p = p0;
     p.split = f32_split(p, f32_vec(a, b, y, p));
-    const dim3 g((p.n + 63) / 64, (p.m + 63) / 64, (unsigned)(p.batch * p.split));
-    hipLaunchKernelGGL((k_matmul_f32_dl<64, 64, 2, 2, 4, 3, 8, false, true>), g, dim3(256), 0, s, (const float *)a,
-                       (const float *)b, (float *)y, p);
+    launch_f32_parts((const float *)a, (const float *)b, (float *)y, p, s);
     const dim3 gr((unsigned)(p.batch * p.m));
     float *fy = (float *)y;
     switch ((p.n + 255) / 256) {
@@ -917,7 +1370,11 @@ hipError_t launch_matmul(int dtype, const void *a, const void *b, void *c, const
             launch_f32_split(fa, fb, fc, q, s);
             return hipGetLastError();
         }
-        // block tile: among the tiles that give each of the 256 CUs two or more blocks (a lone block
+        if (f32_b3(p, p.k)) {
+            launch_f32_b3(fa, fb, fc, p, vec, s);
+            return hipGetLastError();
+        }
+        // K below kB3MinK.  Block tile: among the tiles that give each of the 256 CUs two or more blocks (a lone block
         // per CU leaves its barrier and load latencies unhidden: measured 93 against 104 TF/s for
         // [4096,3072]x[3072,768]), the one whose busiest CU has the least work -- ceil(blocks / 256)
         // blocks, each costing its area over the tile's relative efficiency; 64x64 when none does
@@ -951,9 +1408,7 @@ hipError_t launch_matmul(int dtype, const void *a, const void *b, void *c, const
         // blocks per CU at once (its LDS and its occupancy hint) runs ceil(tiles / (256 r)) rounds, each as long
         // as min(r, tiles per CU) of its tiles, each costing its area over a measured efficiency.  128x128 runs
         // with at most two waves per SIMD (accumulators in AGPRs: 135 TFLOP/s at 4096^3 against 104 with them in
-        // VGPRs for three waves), 128x96 with one or two, the smaller tiles with three or more.  One 128x96 tile
-        // per CU over a long K (at least 2048) keeps that tile: its lone wave per SIMD runs the longest
-        // uninterrupted MFMA stream ([4096,3072]x[3072,768]: 133 against 126 TFLOP/s for 64x64).
+        // VGPRs for three waves), 128x96 with one or two, the smaller tiles with three or more.
         // N of at most 32 (the attention context of 32-wide heads): 128x32 tiles, four waves of 32x32
         // ([8,12,512,512]x[8,12,512,32]: 65 against 43 TFLOP/s for the register-staged kernel's 64x64)
         // (B by columns, p.bt: the register-staged kernel only, never split -- the host checks)
@@ -982,8 +1437,6 @@ hipError_t launch_matmul(int dtype, const void *a, const void *b, void *c, const
                     bc = cost;
                 }
             }
-            const int64_t t96 = tiles_of(dcand[1]);
-            if (t96 > 192 && t96 <= 256 && p.k >= 2048) dt = 1;
             switch (dt) {
             case 0: launch_f32_dl<128, 128, 2, 2, 1, 2>(fa, fb, fc, p, s); break;
             case 1: launch_f32_dl<128, 96, 4, 1, 1, 2>(fa, fb, fc, p, s); break;

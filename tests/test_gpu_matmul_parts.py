@@ -1,0 +1,118 @@
+"""Float MatMul over K ranges of 256 and more, where every operand is split into three bf16 parts and multiplied on
+the bf16 matrix unit (lx_matmul.hip, k_matmul_f32_b3).
+
+Bar: every part product is exact and each of a step's six MFMAs rounds its accumulation once, so a dot product of K
+terms is within (6 ceil(K / 16) + 1) 2^-24 sum_j |a_j b_j| of the exact one (the part products left out weigh 2^-25),
+and within the MatMul bar of 1e-5 sum_j |a_j b_j|."""
+import numpy as np
+import pytest
+
+from onnx_amd import DeviceTensor, HipExecutionProvider as HIP, OpStatus
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    return DeviceTensor.from_numpy(np.asarray(a))
+
+
+def mm(a, b):
+    r = HIP.MatMul(dev(a), dev(b))
+    assert r.Status == OpStatus.Success, r.Message
+    return r.Outputs[0].to_numpy()
+
+
+def check(a, b, got=None):
+    got = (mm(a, b) if got is None else got).astype(np.float64)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    bar = min(1e-5, (6 * -(-a.shape[-1] // 16) + 1) * 2.0 ** -24)
+    err, mag = np.abs(got - a64 @ b64), np.abs(a64) @ np.abs(b64)
+    assert np.all(err <= bar * mag + 2.0 ** -140), float((err / (mag + 1e-300)).max())
+
+
+# every tile (128x128; 128x64; 64x64 several per CU; 64x64 with loading waves), each with whole step pairs, a K tail in
+# 16-byte loads (K % 4 == 0), scalar loads (odd K) and edges in both directions; K ranges of a split product; a batch
+SHAPES = [(256, 256, 128), (4096, 256, 1024), (4096, 384, 384), (1000, 320, 4100), (788, 768, 768), (129, 256, 65),
+          (2000, 260, 2020), (700, 333, 260), (127, 257, 33), (2048, 1001, 1030), (1, 2048, 4096), (300, 1000, 36),
+          (512, 768, 768), (64, 4096, 64), (5, 300, 7)]
+
+
+@pytest.mark.parametrize("m,k,n", SHAPES)
+def test_parts_tiles_and_edges(hip, m, k, n):
+    rng = np.random.default_rng(m + k + n)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    check(a, b)
+
+
+def test_parts_batches(hip):
+    rng = np.random.default_rng(3)
+    for sa, sb in [((3, 1, 130, 256), (1, 2, 256, 132)), ((40, 65, 300), (40, 300, 67))]:
+        check(rng.standard_normal(sa).astype(np.float32), rng.standard_normal(sb).astype(np.float32))
+
+
+@pytest.mark.parametrize("m,k,n", [(260, 256, 516), (256, 333, 70)])
+@pytest.mark.parametrize("kind", ["tiny", "tiny_times_huge", "huge", "mixed", "not_finite"])
+def test_parts_of_extreme_values(hip, m, k, n, kind):
+    """Values whose parts bf16 cannot hold take the fp32 MFMA: subnormal operands, subnormal times huge, values that
+    round to an infinite bf16, rows over 45 decades, and infinities and NaN (the same pattern as float32's)."""
+    rng = np.random.default_rng(7)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    if kind == "tiny":
+        a = (a * 1e-36).astype(np.float32)
+    elif kind == "tiny_times_huge":
+        a, b = (a * 1e-41).astype(np.float32), (b * np.float32(1e20)).astype(np.float32)
+    elif kind == "huge":
+        a[::3, 5] = np.float32(3.4e38)
+        b[5, :] = 0.25
+    elif kind == "mixed":
+        a = (a * 10.0 ** rng.uniform(-30, 15, a.shape)).astype(np.float32)
+    else:
+        a[0, 0], a[2, 5], b[7, 0] = np.nan, np.inf, -np.inf
+        a[3, :], b[:, 2] = 0, 0
+        got = mm(a, b)
+        with np.errstate(all="ignore"):
+            ref = a @ b
+        assert np.array_equal(np.isnan(ref), np.isnan(got))
+        inf = np.isinf(ref)
+        assert np.array_equal(inf, np.isinf(got)) and np.array_equal(ref[inf], got[inf])
+        rows = [i for i in range(m) if i not in (0, 2)]
+        cols = [j for j in range(n) if j != 0]
+        check(a[rows], b[:, cols], got[np.ix_(rows, cols)])
+        return
+    check(a, b)
+
+
+def test_parts_results_do_not_depend_on_the_tile(hip):
+    """The same bits alone and inside a larger product, extreme rows (which take the fp32 MFMA) included (parts of
+    128 tiles of 64x64 or more: fewer split K and sum other ranges)."""
+    rng = np.random.default_rng(11)
+    a, b = rng.standard_normal((4096, 320)).astype(np.float32), rng.standard_normal((320, 1024)).astype(np.float32)
+    a[10] *= np.float32(1e-38)
+    a[70, 3], b[4, 500] = np.inf, np.float32(1e-40)
+    whole = mm(a, b)
+    for rows, cols in [(slice(0, 2048), slice(0, 256)), (slice(0, 1000), slice(448, 1024))]:
+        part = mm(np.ascontiguousarray(a[rows]), np.ascontiguousarray(b[:, cols]))
+        assert np.array_equal(part.view(np.uint32), whole[rows, cols].view(np.uint32))
+
+
+@pytest.mark.parametrize("s,d", [(512, 256), (512, 320), (301, 259)])
+def test_parts_of_a_right_operand_by_columns(hip, s, d):
+    """A transposed right operand folded into the product is read by columns: bit for bit the Transpose and MatMul
+    nodes (128x128 and 64x64 tiles, 16-byte and scalar loads, a K tail)."""
+    import onnx_writer as W
+    from onnx_amd.graph import Model
+    rng = np.random.default_rng(13)
+    ins = {t: rng.standard_normal((2, s, 4, d)).astype(np.float32) for t in "qk"}
+    nodes = [W.node("Transpose", ["q"], ["qt"], "tq", perm=[0, 2, 1, 3]),
+             W.node("Transpose", ["k"], ["kt"], "tk", perm=[0, 2, 3, 1]), W.node("MatMul", ["qt", "kt"], ["y"], "mm")]
+    model = W.model(nodes, [(t, np.float32, v.shape) for t, v in ins.items()], [("y", np.float32, ())], [])
+    d_in = {t: dev(v) for t, v in ins.items()}
+    res = []
+    for fuse in (False, True):
+        g = Model.Load(model)
+        if fuse:
+            assert g.Fuse() == 1 and [x.Op for x in g.Nodes] == ["MatMulPermuted"]
+        assert g.Execute(d_in), g.LastError
+        res.append(g.Output("y").to_numpy())
+    assert np.array_equal(res[0].view(np.uint32), res[1].view(np.uint32))
+    check(ins["q"].transpose(0, 2, 1, 3), ins["k"].transpose(0, 2, 3, 1), res[1])
