@@ -18,7 +18,7 @@ if ARCH != "gfx950":
     # v_rcp_f32 only (tests/native/rcp_check.hip checks every seed on the device)
     raise SystemExit(f"liblonnx_hip is built for gfx950 only (LONNX_OFFLOAD_ARCH={ARCH})")
 
-SOURCES = ["lx_elementwise.hip", "lx_reduce.hip", "lx_softmax.hip", "lx_matmul.hip", "lx_movement.hip", "lx_probe.hip", "lx_api.cpp",
+SOURCES = ["lx_elementwise.hip", "lx_reduce.hip", "lx_softmax.hip", "lx_attention.hip", "lx_matmul.hip", "lx_movement.hip", "lx_probe.hip", "lx_api.cpp",
            "lx_pool.cpp", "lx_graph.cpp", "lx_onnx.cpp"]
 
 # -ffp-contract=off: no FMA contraction of separately rounded float ops.

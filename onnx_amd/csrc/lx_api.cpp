@@ -2010,17 +2010,28 @@ int api_attention(const lx_tensor *Q, const int *q_perm, const lx_tensor *K, con
     permute(q, q_perm);
     permute(k, k_perm);
     permute(v, v_perm);
-    // equal batch axes (no broadcast), heads of at most kAttentionMax: [.., S, D] x [.., D, SK] and [.., S, SK] x
+    // equal batch axes (no broadcast), heads that fit one of the two kernels: [.., S, D] x [.., D, SK] and [.., S, SK] x
     // [.., SK, DV]; otherwise the nodes run (and report any shape error)
     for (int i = 0; i < R - 2; i++)
         if (k.dims[i] != q.dims[i] || v.dims[i] != q.dims[i]) return LX_ERR_NOT_SUPPORTED;
     const int64_t S = q.dims[R - 2], D = q.dims[R - 1], SK = k.dims[R - 1], DV = v.dims[R - 1];
     if (k.dims[R - 2] != D || v.dims[R - 2] != SK) return LX_ERR_NOT_SUPPORTED;
-    for (int64_t e : {S, D, SK, DV})
-        if (e < 1 || e > kAttentionMax) return LX_ERR_NOT_SUPPORTED;
+    bool one_tile = true;
+    for (int64_t e : {S, D, SK, DV}) {
+        if (e < 1 || e > 0x7fffffff) return LX_ERR_NOT_SUPPORTED;
+        one_tile = one_tile && e <= kAttentionMax;
+    }
     int64_t batch = 1;
     for (int i = 0; i < R - 2; i++) batch *= q.dims[i];
     if (batch < 1 || batch > 0x7fffffff) return LX_ERR_NOT_SUPPORTED;
+    AttentionArgs a;
+    memset(&a, 0, sizeof a);
+    a.s = (int)S;
+    a.sk = (int)SK;
+    a.d = (int)D;
+    a.dv = (int)DV;
+    a.batch = batch;
+    if (!one_tile && !attention_long_fits(a)) return LX_ERR_NOT_SUPPORTED;
     // the Softmax over the scores' last axis with the scale and mask in its kernel, as run_softmax takes them
     int64_t sdims[LX_MAX_RANK];
     for (int i = 0; i < R - 2; i++) sdims[i] = q.dims[i];
@@ -2050,18 +2061,11 @@ int api_attention(const lx_tensor *Q, const int *q_perm, const lx_tensor *K, con
         cstr[y_perm ? y_perm[i] : i] = ys;
         ys *= ydims[i];
     }
-    AttentionArgs a;
-    memset(&a, 0, sizeof a);
     a.q = (const float *)Q->data;
     a.k = (const float *)K->data;
     a.v = (const float *)V->data;
     a.y = (float *)Y->data;
-    a.s = (int)S;
-    a.sk = (int)SK;
-    a.d = (int)D;
-    a.dv = (int)DV;
     a.nbatch = R - 2;
-    a.batch = batch;
     for (int i = 0; i < R - 2; i++) {
         a.bdims[i] = q.dims[i];
         a.q_bstr[i] = q.str[i];
@@ -2078,7 +2082,7 @@ int api_attention(const lx_tensor *Q, const int *q_perm, const lx_tensor *K, con
     a.mask_rows = sa.mask_rows;
     a.scale = scale ? (const float *)scale->data : nullptr;
     a.scale_div = scale_div;
-    HIPCHECK(launch_attention(a, g.stream), "Attention");
+    HIPCHECK(one_tile ? launch_attention(a, g.stream) : launch_attention_long(a, g.stream), "Attention");
     return LX_OK;
 }
 }  // namespace lx

@@ -104,6 +104,28 @@ __device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv &f) {
     return (__umulhi(n, f.m) + n) >> f.s;
 }
 
+// Mask row offset: the row index decomposed over the mask's row axes
+// (innermost first).  NOUT >= 0 is the compile-time axis count, -1 = runtime.
+template <int NOUT>
+__device__ __forceinline__ int64_t mask_row_offset(uint32_t row, const NdLayout &L) {
+    int64_t off = 0;
+    if constexpr (NOUT >= 0) {
+#pragma unroll
+        for (int d = 0; d < NOUT; d++) {
+            uint32_t q = fdiv(row, L.odiv[d]);
+            off += (int64_t)(row - q * L.odiv[d].d) * L.a_str[d];
+            row = q;
+        }
+    } else {
+        for (int d = 0; d < L.nouter; d++) {
+            uint32_t q = fdiv(row, L.odiv[d]);
+            off += (int64_t)(row - q * L.odiv[d].d) * L.a_str[d];
+            row = q;
+        }
+    }
+    return off;
+}
+
 // ---------------------------------------------------------------------------
 // Wave64 reductions (butterfly over __shfl_xor; fixed order -> deterministic).
 // ---------------------------------------------------------------------------

@@ -72,28 +72,6 @@ __device__ __forceinline__ T div_row(T e, T s, T rs) {
     else return e / s;
 }
 
-// Mask row offset: the row index decomposed over the mask's row axes
-// (innermost first).  NOUT >= 0 is the compile-time axis count, -1 = runtime.
-template <int NOUT>
-__device__ __forceinline__ int64_t mask_row_offset(uint32_t row, const NdLayout &L) {
-    int64_t off = 0;
-    if constexpr (NOUT >= 0) {
-#pragma unroll
-        for (int d = 0; d < NOUT; d++) {
-            uint32_t q = fdiv(row, L.odiv[d]);
-            off += (int64_t)(row - q * L.odiv[d].d) * L.a_str[d];
-            row = q;
-        }
-    } else {
-        for (int d = 0; d < L.nouter; d++) {
-            uint32_t q = fdiv(row, L.odiv[d]);
-            off += (int64_t)(row - q * L.odiv[d].d) * L.a_str[d];
-            row = q;
-        }
-    }
-    return off;
-}
-
 // Loads one row's vectors (and, with a mask, the mask vectors it adds): the
 // mask loads go first so that a wave waiting for them never waits for loads
 // issued after them.
