@@ -973,13 +973,20 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
         mm_epilogue<MT, NT, false, GELU>(acc, C, p, co, row0 + wr, col0 + wc, l, tab);
 }
 
-constexpr int kB3MinK = 256;
+constexpr int kB3MinK = 256, kB3LoneK = 512;
 // Whether a K range of kr goes to k_matmul_f32_b3: kB3MinK or more, N above 32 (a context product of 32-wide heads is
 // bound by its loads: [96,512,512]x[96,512,32] 24 us on the fp32 MFMA, 26 in parts), and strides whose offsets within
-// a tile and a step stay below 2^31 bytes (rows of up to 8 MB; longer ones keep the fp32 MFMA).
+// a tile and a step stay below 2^31 bytes (rows of up to 8 MB; longer ones keep the fp32 MFMA).  A range below kB3LoneK
+// whose blocks (of one matrix in a grouped launch, which has to give the bits of its single products) find a CU each
+// keeps the fp32 MFMA too: the parts' first stage and last check cost 1.2 us more than a block of so few steps gains
+// ([640,1536]x[1536,384] 14.9 against 13.2 us a call, six batches of 384^3 11.8 against 10.2; [1024,512]x[512,512],
+// the first on the other side, 11.3 against 11.2).
 static bool f32_b3(const MatMulArgs &p, int kr) {
     const int64_t lim = (int64_t)1 << 21;
-    return kr >= kB3MinK && p.n > 32 && p.lda <= lim && p.ldb <= lim && p.k <= (1 << 24);
+    if (kr < kB3MinK || p.n <= 32 || p.lda > lim || p.ldb > lim || p.k > (1 << 24)) return false;
+    const int64_t blocks = (((int64_t)p.m + 63) / 64) * (((int64_t)p.n + 63) / 64) * (p.k / kr) *
+                           (p.split_per_matrix ? 1 : p.batch);
+    return kr >= kB3LoneK || blocks > 256;
 }
 
 // The block tile: the least estimated time.  A tile's step of 16 k takes `lone` us when its block has a CU to itself

@@ -34,7 +34,8 @@ def check(a, b, got=None):
 # 16-byte loads (K % 4 == 0), scalar loads (odd K) and edges in both directions; K ranges of a split product; a batch
 SHAPES = [(256, 256, 128), (4096, 256, 1024), (4096, 384, 384), (1000, 320, 4100), (788, 768, 768), (129, 256, 65),
           (2000, 260, 2020), (700, 333, 260), (127, 257, 33), (2048, 1001, 1030), (1, 2048, 4096), (300, 1000, 36),
-          (512, 768, 768), (64, 4096, 64), (5, 300, 7)]
+          (512, 768, 768), (64, 4096, 64), (5, 300, 7),
+          (1024, 512, 512), (1100, 516, 512), (100, 600, 70), (1100, 384, 960)]  # a CU per tile: from K = 512
 
 
 @pytest.mark.parametrize("m,k,n", SHAPES)
@@ -46,11 +47,11 @@ def test_parts_tiles_and_edges(hip, m, k, n):
 
 def test_parts_batches(hip):
     rng = np.random.default_rng(3)
-    for sa, sb in [((3, 1, 130, 256), (1, 2, 256, 132)), ((40, 65, 300), (40, 300, 67))]:
+    for sa, sb in [((3, 1, 130, 256), (1, 2, 256, 132)), ((70, 65, 300), (70, 300, 67))]:
         check(rng.standard_normal(sa).astype(np.float32), rng.standard_normal(sb).astype(np.float32))
 
 
-@pytest.mark.parametrize("m,k,n", [(260, 256, 516), (256, 333, 70)])
+@pytest.mark.parametrize("m,k,n", [(260, 512, 516), (256, 533, 70), (1090, 333, 1000)])
 @pytest.mark.parametrize("kind", ["tiny", "tiny_times_huge", "huge", "mixed", "not_finite"])
 def test_parts_of_extreme_values(hip, m, k, n, kind):
     """Values whose parts bf16 cannot hold take the fp32 MFMA: subnormal operands, subnormal times huge, values that
@@ -83,19 +84,19 @@ def test_parts_of_extreme_values(hip, m, k, n, kind):
 
 
 def test_parts_results_do_not_depend_on_the_tile(hip):
-    """The same bits alone and inside a larger product, extreme rows (which take the fp32 MFMA) included (parts of
-    128 tiles of 64x64 or more: fewer split K and sum other ranges)."""
+    """The same bits alone and inside a larger product, extreme rows (which take the fp32 MFMA) included (parts of more
+    than 256 tiles of 64x64: fewer keep the fp32 MFMA at this K, or split K and sum other ranges)."""
     rng = np.random.default_rng(11)
     a, b = rng.standard_normal((4096, 320)).astype(np.float32), rng.standard_normal((320, 1024)).astype(np.float32)
     a[10] *= np.float32(1e-38)
     a[70, 3], b[4, 500] = np.inf, np.float32(1e-40)
     whole = mm(a, b)
-    for rows, cols in [(slice(0, 2048), slice(0, 256)), (slice(0, 1000), slice(448, 1024))]:
+    for rows, cols in [(slice(0, 2048), slice(0, 576)), (slice(0, 2200), slice(448, 1024))]:
         part = mm(np.ascontiguousarray(a[rows]), np.ascontiguousarray(b[:, cols]))
         assert np.array_equal(part.view(np.uint32), whole[rows, cols].view(np.uint32))
 
 
-@pytest.mark.parametrize("s,d", [(512, 256), (512, 320), (301, 259)])
+@pytest.mark.parametrize("s,d", [(512, 256), (512, 320), (301, 515)])
 def test_parts_of_a_right_operand_by_columns(hip, s, d):
     """A transposed right operand folded into the product is read by columns: bit for bit the Transpose and MatMul
     nodes (128x128 and 64x64 tiles, 16-byte and scalar loads, a K tail)."""
