@@ -1069,6 +1069,115 @@ static void launch_f32_parts(const float *a, const float *b, float *c, const Mat
         hipLaunchKernelGGL((k_matmul_f32_dl<64, 64, 2, 2, 4, 3, 8, false, true>), g, dim3(256), 0, s, a, b, c, p);
 }
 
+// ---------------------------------------------------------------------------
+// float, split products of few rows (a short query's projections): one launch
+// ---------------------------------------------------------------------------
+// The K ranges of a split product and their ordered sum in one block, on the VALU: v_mfma_f32_32x32x2f32 is two fused
+// multiply-adds per result, the lower lanes' k first (checked bit for bit over 200,000 results of every magnitude), so
+// a chain of v_fma_f32 in the fp32 kernels' order gives the partial products' bits without the rows of zeros that the
+// MFMA would multiply.  A block takes kSmallR rows and kSmallC columns, a lane one column of one range (four ranges per
+// wave): its 64 elements of the right operand are loaded at once, one memory latency for the whole of K; the rows come
+// from LDS, each range padded by four floats (the four ranges of a wave read different banks).  The partials then meet
+// in LDS and are summed in range order with the epilogue, exactly as k_matmul_split_sum does.
+// Bound: launches and memory latency.  5.1 us a product ([8,1536]x[1536,384] and the like) in place of 4.3 for the
+// tiles and 3.7 to 5.4 for the sum; a captured encoder of 12 layers of 384 at 8 tokens 510 -> 400 us, at 32 530 -> 430,
+// at 64 584 -> 512.
+constexpr int kSmallR = 4, kSmallC = 16, kSmallRanges = 64;
+
+template <bool GELU>
+__global__ __launch_bounds__(1024) void k_matmul_small(const float *__restrict__ A, const float *__restrict__ B,
+                                                       float *__restrict__ C, MatMulArgs p) {
+    extern __shared__ float sh[];  // rows [kSmallR][split * (range + 4)], then partials [split][kSmallR][kSmallC]
+    __shared__ ExpTable tab;
+    if constexpr (GELU) exp_table_fill(tab);
+    constexpr int RL = 64;  // the length of a range
+    const int M = p.m, N = p.n, R = p.split, LD = R * (RL + 4);
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int col0 = blockIdx.x * kSmallC, row0 = blockIdx.y * kSmallR;
+    int64_t ao = 0, bo = 0, co = 0;
+    if (p.nbatch) batch_offsets(p.batch_base + blockIdx.z, p, &ao, &bo, &co);
+    // the rows first (they are waited for first): each wave its own four ranges, lane l 16 bytes of range l / 16
+    constexpr int RW = 64 / kSmallC;  // ranges per wave
+    const int range = min(w * RW + l / kSmallC, R - 1), c = l % kSmallC;
+    v4f av[kSmallR];
+    const float *Ar = A + ao + range * RL + 4 * c;
+#pragma unroll
+    for (int r = 0; r < kSmallR; r++) av[r] = *reinterpret_cast<const v4f *>(Ar + (int64_t)min(row0 + r, M - 1) * p.lda);
+    sched_fence();
+    const float *Bc = B + bo + (int64_t)range * RL * p.ldb + min(col0 + c, N - 1);
+    float b[RL];
+#pragma unroll
+    for (int k = 0; k < RL; k++) b[k] = Bc[(int64_t)k * p.ldb];
+    sched_fence();
+    // the outputs' bias and residual with them
+    const int orow = row0 + (int)threadIdx.x / kSmallC, ocol = col0 + (int)threadIdx.x % kSmallC;
+    const bool out = threadIdx.x < kSmallR * kSmallC && orow < M && ocol < N;
+    const int64_t bz = p.batch_base + blockIdx.z;
+    const float bias = out && p.bias ? p.bias[bz * p.bias_bstr + ocol] : 0.f;
+    const float res = out && p.res ? p.res[bz * (int64_t)M * N + (int64_t)orow * N + ocol] : 0.f;
+    float *as = sh + range * (RL + 4);
+#pragma unroll
+    for (int r = 0; r < kSmallR; r++) *reinterpret_cast<v4f *>(as + r * LD + 4 * c) = av[r];
+    // a wave reads only the ranges it wrote
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    float acc[kSmallR];
+#pragma unroll
+    for (int r = 0; r < kSmallR; r++) acc[r] = 0.f;
+#pragma unroll
+    for (int s = 0; s < RL; s += 16)
+#pragma unroll
+        for (int r = 0; r < kSmallR; r++) {
+            v4f a[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) a[i] = *reinterpret_cast<const v4f *>(as + r * LD + s + 4 * i);
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                acc[r] = __builtin_fmaf(a[j / 4][j % 4], b[s + j], acc[r]);
+                acc[r] = __builtin_fmaf(a[2 + j / 4][j % 4], b[s + 8 + j], acc[r]);
+            }
+        }
+    float *part = sh + kSmallR * LD;  // (ranges past the last: the last one's values again)
+#pragma unroll
+    for (int r = 0; r < kSmallR; r++) part[(range * kSmallR + r) * kSmallC + c] = acc[r];
+    __syncthreads();
+    if (!out) return;
+    constexpr int kOut = kSmallR * kSmallC, kChunk = 8;
+    const float *P = part + threadIdx.x;
+    float v = P[0];
+    for (int g0 = 1; g0 < R; g0 += kChunk) {
+        float x[kChunk];
+#pragma unroll
+        for (int g = 0; g < kChunk; g++) x[g] = P[min(g0 + g, R - 1) * kOut];
+#pragma unroll
+        for (int g = 0; g < kChunk; g++)
+            if (g0 + g < R) v = v + x[g];
+    }
+    if (p.bias) v = v + bias;
+    if (p.res) v = v + res;
+    if constexpr (GELU) {
+        v = gelu_erf_lx(v, tab);
+    }
+    C[co + (int64_t)orow * p.ldc + ocol] = v;
+}
+
+// Whether a product of `split` ranges goes to k_matmul_small: ranges of 64 (K below 128 times the ranges the chip has
+// room for), at most kSmallRanges of them (a block of 16 waves), and at most kSmallM rows: every four rows read the
+// right operand again from L2, and above a tile of 64 the ranges of a long K are no longer 64.  Blocks of eight rows
+// measured slower up to 64 rows (32 rows: 473 against 430 us for the 12-layer encoder).
+constexpr int kSmallM = 64;
+static bool f32_small(const MatMulArgs &p, int split) {
+    return split > 1 && split <= kSmallRanges && p.k / split == 64 && p.m <= kSmallM && !p.bt;
+}
+static void launch_f32_small(const float *a, const float *b, float *c, const MatMulArgs &p, hipStream_t s) {
+    const dim3 g((p.n + kSmallC - 1) / kSmallC, (p.m + kSmallR - 1) / kSmallR, (unsigned)p.batch);
+    const dim3 blk(64 * ((p.split + 64 / kSmallC - 1) / (64 / kSmallC)));
+    const size_t lds = (size_t)(kSmallR * (p.k + 4 * p.split) + p.split * kSmallR * kSmallC) * sizeof(float);
+    if (p.gelu) hipLaunchKernelGGL(k_matmul_small<true>, g, blk, lds, s, a, b, c, p);
+    else hipLaunchKernelGGL(k_matmul_small<false>, g, blk, lds, s, a, b, c, p);
+}
+
 // Split K (p.split ranges, p.part holding the partials): 64x64 tiles, then the ordered sum with the epilogue.
 static void launch_f32_split(const float *a, const float *b, float *c, const MatMulArgs &p, hipStream_t s) {
     launch_f32_parts(a, b, c, p, s);
@@ -1348,7 +1457,7 @@ hipError_t launch_matmul_ln(const void *a, const void *b, void *y, const MatMulA
 int64_t matmul_part_bytes(int dtype, const void *a, const void *b, const void *c, const MatMulArgs &p) {
     if (dtype != kFloat || p.m == 0 || p.n == 0 || p.batch == 0) return 0;
     const int r = f32_split(p, f32_vec(a, b, c, p));
-    return r > 1 ? (int64_t)r * p.batch * p.m * p.n * (int64_t)sizeof(float) : 0;
+    return r > 1 && !f32_small(p, r) ? (int64_t)r * p.batch * p.m * p.n * (int64_t)sizeof(float) : 0;
 }
 
 hipError_t launch_matmul(int dtype, const void *a, const void *b, void *c, const MatMulArgs &p0, hipStream_t s) {
@@ -1370,6 +1479,12 @@ hipError_t launch_matmul(int dtype, const void *a, const void *b, void *c, const
         const float *fa = (const float *)a, *fb = (const float *)b;
         float *fc = (float *)c;
         const int split = f32_split(p, vec);
+        if (f32_small(p, split)) {
+            MatMulArgs q = p;
+            q.split = split;
+            launch_f32_small(fa, fb, fc, q, s);
+            return hipGetLastError();
+        }
         if (split > 1) {
             if (!p.part || p.bt) return hipErrorInvalidValue;  // the caller sizes it with matmul_part_bytes
             MatMulArgs q = p;
