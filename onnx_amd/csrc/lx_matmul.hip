@@ -11,8 +11,8 @@
 //         one K step ahead (k_matmul_f32).  Block tiles from 64x64 to 128x128
 //         chosen per shape, K step 16, four waves.
 // double: v_mfma_f64_16x16x4f64, 64x64 block tile, four waves of 32x32.
-// int32 : exact two's-complement multiply-add on the VALU (no int32 MFMA),
-//         16x16 LDS tiles.
+// int32 : exact two's-complement products as ten int8 digit products on
+//         v_mfma_i32_32x32x32_i8 (small products of K up to 96: on the VALU).
 // Batches: the leading (broadcast) axes are decomposed per block with
 // per-operand element strides, 0 on broadcast axes (no materialisation).
 // Layout of the MFMA operands and results checked on the device:
@@ -1331,10 +1331,207 @@ static void launch_f64(const double *a, const double *b, double *c, const MatMul
 }
 
 // ---------------------------------------------------------------------------
-// int32: exact wrapping multiply-add (C# unchecked int arithmetic)
+// int32: exact wrapping multiply-add (C# unchecked int arithmetic) on the int8 matrix unit
 // ---------------------------------------------------------------------------
+// Modulo 2^32 an int32 is four signed base-256 digits, x = d0 + 2^8 d1 + 2^16 d2 + 2^24 d3, -128 <= d <= 127: the
+// bytes of (x + 0x80808080) ^ 0x80808080.  A product is then the ten digit products of weight below 2^32, those of one
+// weight summed in one int32 accumulator by v_mfma_i32_32x32x32_i8: exact below 2^31, i.e. for 2^15 k (up to four
+// products of 2^14 each per k), so every kFoldK the four accumulators are folded into the wrapping result.
+//
+// k_matmul_i32: 64x64 tile, four waves of 32x32 (four accumulators each), K steps of 64.  Elements go from global memory
+// to registers one step ahead, are split (two instructions, then a 4x4 byte transpose) and written to LDS as four digit
+// planes, [row][64 k] bytes with rows 80 bytes apart (the 16-byte fragment reads are free of bank conflicts); two
+// stages, one barrier per step.  Past M, N and K loads clamp; elements past K are zero.
+// Bound: the latency of a step's loads and its splitting (about 1.5 us a step), not the matrix unit: 12 products of
+// 512^3 206 us on the VALU (16 TOPS), 36 here (90 TOPS).
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x4u __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes at 4-byte alignment: one load
+constexpr int kI32Fold = 16384;
+
+// sixteen elements k .. k + 15 of a row of K (clamped to the row)
+__device__ __forceinline__ void i32_load_row(const int32_t *row, int k, int K, uint32_t (&x)[16]) {
+    if (k + 16 <= K) {
+#pragma unroll
+        for (int g = 0; g < 16; g += 4) {
+            const i32x4u v = *reinterpret_cast<const i32x4u *>(row + k + g);
+#pragma unroll
+            for (int e = 0; e < 4; e++) x[g + e] = (uint32_t)v[e];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 16; e++) x[e] = (uint32_t)row[min(k + e, K - 1)];
+    }
+}
+// and of a column, ldb apart
+__device__ __forceinline__ void i32_load_col(const int32_t *col, int64_t ldb, int k, int K, uint32_t (&y)[16]) {
+#pragma unroll
+    for (int e = 0; e < 16; e++) y[e] = (uint32_t)col[(int64_t)min(k + e, K - 1) * ldb];
+}
+// the digits of sixteen elements (zero from element `left` on), one 16-byte row piece per plane
+template <int PLANE>
+__device__ __forceinline__ void i32_store_digits(const uint32_t (&v)[16], int left, char *d) {
+    i32x4 dig[4];
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        uint32_t q[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) q[e] = 4 * g + e < left ? (v[4 * g + e] + 0x80808080u) ^ 0x80808080u : 0u;
+        const uint32_t a01 = __builtin_amdgcn_perm(q[1], q[0], 0x05010400u);  // bytes 0, 0', 1, 1'
+        const uint32_t b01 = __builtin_amdgcn_perm(q[1], q[0], 0x07030602u);  // bytes 2, 2', 3, 3'
+        const uint32_t a23 = __builtin_amdgcn_perm(q[3], q[2], 0x05010400u);
+        const uint32_t b23 = __builtin_amdgcn_perm(q[3], q[2], 0x07030602u);
+        dig[0][g] = (int)__builtin_amdgcn_perm(a23, a01, 0x05040100u);
+        dig[1][g] = (int)__builtin_amdgcn_perm(a23, a01, 0x07060302u);
+        dig[2][g] = (int)__builtin_amdgcn_perm(b23, b01, 0x05040100u);
+        dig[3][g] = (int)__builtin_amdgcn_perm(b23, b01, 0x07060302u);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) *reinterpret_cast<i32x4 *>(d + i * PLANE) = dig[i];
+}
+// one 32x32 tile over 32 k: the fragments of the four planes of A at fa and of B at fb
+template <int PLANE>
+__device__ __forceinline__ void i32_mfma10(const char *fa, const char *fb, i32x16 (&acc)[4]) {
+    i32x4 a[4], b[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        a[i] = *reinterpret_cast<const i32x4 *>(fa + i * PLANE);
+        b[i] = *reinterpret_cast<const i32x4 *>(fb + i * PLANE);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; i + j < 4; j++) acc[i + j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(b[j], a[i], acc[i + j], 0, 0, 0);
+}
+__device__ __forceinline__ void i32_fold(i32x16 (&acc)[4], uint32_t (&total)[16]) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        total[r] += (uint32_t)acc[0][r] + ((uint32_t)acc[1][r] << 8) + ((uint32_t)acc[2][r] << 16) + ((uint32_t)acc[3][r] << 24);
+        acc[0][r] = acc[1][r] = acc[2][r] = acc[3][r] = 0;
+    }
+}
+
 __global__ __launch_bounds__(256) void k_matmul_i32(const int32_t *__restrict__ A, const int32_t *__restrict__ B,
-                                                    int32_t *__restrict__ C, MatMulArgs p) {
+                                                    int32_t *__restrict__ C, MatMulArgs p, int vc) {
+    constexpr int KB = 64, LD = KB + 16, PLANE = 64 * LD;
+    __shared__ __attribute__((aligned(16))) char sm[2][8 * PLANE];  // digit planes of A, then of B
+    const int M = p.m, N = p.n, K = p.k;
+    const int t = threadIdx.x, l = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int row0 = blockIdx.y * 64, col0 = blockIdx.x * 64;
+    int64_t ao, bo, co;
+    batch_offsets(p.batch_base + blockIdx.z, p, &ao, &bo, &co);
+    // this thread's elements of a step: 16 k of one row of A, 16 k of one column of B
+    const int ak = t % 4 * 16, bk = w * 16;
+    const int32_t *Ar = A + ao + (int64_t)min(row0 + t / 4, M - 1) * p.lda;
+    const int32_t *Bc = B + bo + min(col0 + l, N - 1);
+    const int aw = t / 4 * LD + ak, bw = 4 * PLANE + l * LD + bk;
+    const int fa = (w / 2 * 32 + l % 32) * LD + l / 32 * 16, fb = 4 * PLANE + (w % 2 * 32 + l % 32) * LD + l / 32 * 16;
+    uint32_t x[16], y[16], total[16];
+    i32x16 acc[4];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        total[r] = 0;
+        acc[0][r] = acc[1][r] = acc[2][r] = acc[3][r] = 0;
+    }
+    if (K > 0) {
+        i32_load_row(Ar, ak, K, x);
+        i32_load_col(Bc, p.ldb, bk, K, y);
+    }
+    for (int k0 = 0; k0 < K; k0 += KB) {
+        char *st = sm[k0 / KB & 1];
+        i32_store_digits<PLANE>(x, K - k0 - ak, st + aw);
+        i32_store_digits<PLANE>(y, K - k0 - bk, st + bw);
+        // (one barrier per step: a wave writes this stage again only after the next step's barrier, which every wave
+        // reaches with its reads of it done)
+        __syncthreads();
+        if (k0 + KB < K) {
+            i32_load_row(Ar, k0 + KB + ak, K, x);
+            i32_load_col(Bc, p.ldb, k0 + KB + bk, K, y);
+        }
+#pragma unroll
+        for (int u = 0; u < KB; u += 32) i32_mfma10<PLANE>(st + fa + u, st + fb + u, acc);
+        if (k0 % kI32Fold == kI32Fold - KB) i32_fold(acc, total);
+    }
+    i32_fold(acc, total);
+    const int row = row0 + w / 2 * 32 + l % 32;
+    if (row >= M) return;
+    int32_t *Cr = C + co + (int64_t)row * p.ldc;
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        const int col = col0 + w % 2 * 32 + 8 * g + l / 32 * 4;
+        if (vc) {
+            if (col < N) *reinterpret_cast<i32x4 *>(Cr + col) = i32x4{(int)total[4 * g], (int)total[4 * g + 1], (int)total[4 * g + 2], (int)total[4 * g + 3]};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (col + e < N) Cr[col + e] = (int32_t)total[4 * g + e];
+        }
+    }
+}
+
+// Few tiles: 32x32 tiles whose K is dealt out to the block's waves in steps of 32, every wave splitting and multiplying
+// its own steps from its own planes (no barrier), the waves' sums joined in LDS.
+constexpr int kI32Waves = 8, kI32FewLd = 48, kI32FewPlane = 32 * kI32FewLd;  // rows 48 bytes apart: free of conflicts
+__global__ __launch_bounds__(kI32Waves * 64) void k_matmul_i32_few(const int32_t *__restrict__ A, const int32_t *__restrict__ B,
+                                                                  int32_t *__restrict__ C, MatMulArgs p) {
+    constexpr int KB = 32, LD = kI32FewLd, PLANE = kI32FewPlane;
+    extern __shared__ __attribute__((aligned(16))) char dyn[];
+    const int M = p.m, N = p.n, K = p.k;
+    const int t = threadIdx.x, l = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6), nw = blockDim.x >> 6;
+    const int row0 = blockIdx.y * 32, col0 = blockIdx.x * 32;
+    int64_t ao, bo, co;
+    batch_offsets(p.batch_base + blockIdx.z, p, &ao, &bo, &co);
+    const int ak = l % 2 * 16, bk = l / 32 * 16;
+    const int32_t *Ar = A + ao + (int64_t)min(row0 + l / 2, M - 1) * p.lda;
+    const int32_t *Bc = B + bo + min(col0 + l % 32, N - 1);
+    char *st = dyn + w * 8 * PLANE;
+    uint32_t x[16], y[16], total[16];
+    i32x16 acc[4];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        total[r] = 0;
+        acc[0][r] = acc[1][r] = acc[2][r] = acc[3][r] = 0;
+    }
+    int k0 = w * KB, n = 0;
+    if (k0 < K) {
+        i32_load_row(Ar, k0 + ak, K, x);
+        i32_load_col(Bc, p.ldb, k0 + bk, K, y);
+    }
+    auto wave_sync = []() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    for (; k0 < K; k0 += nw * KB) {
+        i32_store_digits<PLANE>(x, K - k0 - ak, st + l / 2 * LD + ak);
+        i32_store_digits<PLANE>(y, K - k0 - bk, st + 4 * PLANE + l % 32 * LD + bk);
+        wave_sync();
+        if (k0 + nw * KB < K) {
+            i32_load_row(Ar, k0 + nw * KB + ak, K, x);
+            i32_load_col(Bc, p.ldb, k0 + nw * KB + bk, K, y);
+        }
+        i32_mfma10<PLANE>(st + l % 32 * LD + l / 32 * 16, st + 4 * PLANE + l % 32 * LD + l / 32 * 16, acc);
+        wave_sync();
+        if (++n % (kI32Fold / KB) == 0) i32_fold(acc, total);
+    }
+    i32_fold(acc, total);
+    // [wave][r][lane], r 65 words apart; then output i of the tile is row i / 32, column i % 32
+    uint32_t *sum = (uint32_t *)dyn;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; r++) sum[(w * 16 + r) * 65 + l] = total[r];
+    __syncthreads();
+    for (int i = t; i < 1024; i += blockDim.x) {
+        const int row = i / 32, col = i % 32, s0 = (4 * (col / 8) + col % 4) * 65 + row + col / 4 % 2 * 32;
+        uint32_t v = 0;
+        for (int g = 0; g < nw; g++) v += sum[g * 16 * 65 + s0];
+        if (row0 + row < M && col0 + col < N) C[co + (int64_t)(row0 + row) * p.ldc + col0 + col] = (int32_t)v;
+    }
+}
+
+// Short K: the multiply-adds on the VALU, an output per thread.
+__global__ __launch_bounds__(256) void k_matmul_i32_short(const int32_t *__restrict__ A, const int32_t *__restrict__ B,
+                                                          int32_t *__restrict__ C, MatMulArgs p) {
     __shared__ uint32_t As[16][17], Bs[16][17];
     const int M = p.m, N = p.n, K = p.k;
     const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
@@ -1353,6 +1550,35 @@ __global__ __launch_bounds__(256) void k_matmul_i32(const int32_t *__restrict__ 
         __syncthreads();
     }
     if (row < M && col < N) C[co + (int64_t)row * p.ldc + col] = (int32_t)acc;
+}
+
+// Which kernel (us a call).  K of one step of 16, and K up to kI32ShortK of at most kI32ShortWork multiply-adds: the
+// VALU, done before a split pays (12 products of 32^3 4.2 against 6.3 in 32x32 tiles, 64^3 4.2 / 5.0, 12 of 70^3 5.0 /
+// 5.6, [768,16]x[16,768] 4.4 / 4.9 in 64x64 tiles; past it 12 of 100^3 6.4 / 5.4, [768,64]x[64,768] 8.1 / 4.7).  Then, of
+// at most kI32FewTiles tiles of 64x64 (half the CUs): 32x32 tiles with K over the waves ([1,768]x[768,768] 22.5 on the
+// VALU, 21.4 in 64x64 tiles, 7.5; 384^3 16.1 / 12.1 / 5.5; six of 250^3 17.9 / 11.1 / 9.4).  More tiles take the 64x64
+// form, which reads the operands half as often (six of 384^3, 216 tiles: 51.5 / 13.5 / 18.8; 12 of 256^3, 192 tiles:
+// 31.1 / 10.0 / 12.2; 12 of 512^3: 205 / 36 / 60).
+constexpr int kI32FewTiles = 128, kI32ShortK = 96;
+constexpr int64_t kI32ShortWork = (int64_t)1 << 23;
+static void launch_i32(const int32_t *a, const int32_t *b, int32_t *c, const MatMulArgs &p, hipStream_t s) {
+    const int64_t tiles = (((int64_t)p.m + 63) / 64) * (((int64_t)p.n + 63) / 64) * p.batch;
+    if (p.k <= 16 || (p.k <= kI32ShortK && (int64_t)p.m * p.n <= kI32ShortWork / p.k / p.batch)) {
+        const dim3 g((p.n + 15) / 16, (p.m + 15) / 16, (unsigned)p.batch);
+        hipLaunchKernelGGL(k_matmul_i32_short, g, dim3(256), 0, s, a, b, c, p);
+        return;
+    }
+    if (tiles <= kI32FewTiles) {
+        const int nw = min(kI32Waves, (p.k + 31) / 32);
+        const dim3 g((p.n + 31) / 32, (p.m + 31) / 32, (unsigned)p.batch);
+        hipLaunchKernelGGL(k_matmul_i32_few, g, dim3(64 * nw), (size_t)nw * 8 * kI32FewPlane, s, a, b, c, p);
+        return;
+    }
+    // 16-byte stores of C's rows
+    bool vc = p.n % 4 == 0 && p.ldc % 4 == 0 && (uintptr_t)c % 16 == 0;
+    for (int d = 0; d < p.nbatch; d++) vc = vc && p.c_bstr[d] % 4 == 0;
+    const dim3 g((p.n + 63) / 64, (p.m + 63) / 64, (unsigned)p.batch);
+    hipLaunchKernelGGL(k_matmul_i32, g, dim3(256), 0, s, a, b, c, p, (int)vc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1584,8 +1810,7 @@ hipError_t launch_matmul(int dtype, const void *a, const void *b, void *c, const
         else if (tiles(64) >= 256) launch_f64<64, 64>(da, db, dc, p, s);
         else launch_f64<32, 32>(da, db, dc, p, s);
     } else if (dtype == kInt32) {
-        dim3 g((p.n + 15) / 16, (p.m + 15) / 16, (unsigned)p.batch);
-        hipLaunchKernelGGL(k_matmul_i32, g, dim3(256), 0, s, (const int32_t *)a, (const int32_t *)b, (int32_t *)c, p);
+        launch_i32((const int32_t *)a, (const int32_t *)b, (int32_t *)c, p, s);
     } else {
         return hipErrorInvalidValue;
     }
