@@ -622,14 +622,18 @@ static void launch_f32_dl(const float *a, const float *b, float *c, const MatMul
 // 128).  Shorter ranges stay on the fp32 MFMA: they are bound by launches and loads ([667,384]x[384,384] in ranges of
 // 128 ran slower in parts).  The choice is by the length of the K range alone, so that a product is the same bits in every tile, fused or not, folded or not.
 //
-// What the parts cannot hold goes to the fp32 MFMA, element by element: values that are not finite (or round to an
-// infinite bf16) make the result not finite, and parts below 2^-133 are lost, which a result smaller than 2^-90 of
-// its row's and column's largest operand can show.  Each thread keeps the largest magnitude it loaded of its row and
-// column; a wave holding such a result runs that 32x32 tile again from global memory (f32_tile) and takes those
-// elements from it.  (A row or column of zeros needs no second run: its results are zero.)
+// What the parts cannot hold goes to the fp32 MFMA, element by element: a result that is not finite (a value that is
+// not, or rounds to an infinite bf16); a result smaller than 2^-96 of its column's largest operand where its row holds
+// a nonzero value below 2^-109 (parts below 2^-133 are lost: 2^-134 of the operand per product), and the other way
+// round; and a result below 2^-120 that is not zero or has no product of 2^-120 in its row and column (the small part
+// products are lost below float32's range).  Each thread keeps the largest magnitude it loaded of its row and column
+// and the smallest but zero; a wave holding such a result runs that 32x32 tile again from global memory (f32_tile) and
+// takes those elements from it.  A zero or small result alone says nothing: products of integers, of sparse operands
+// or of values of 1e-24 take the time of any others ([4096,768]x[768,768] of values -8..8 ran 186 us when every zero
+// ran again, 33 now; the smallest magnitudes cost normal data 1 to 3%).
 //
 // Bound: the matrix unit (register-only, 340 TFLOP/s of float32 products at the clock it holds), then the issue slots
-// of the splitting (11 VALU instructions per pair of elements) and of LDS, so each element is split once per block,
+// of the splitting (15 VALU instructions per pair of elements) and of LDS, so each element is split once per block,
 // on its way from global memory to LDS, and the splitting, the LDS accesses and the loads are dealt out between the
 // MFMAs one by one (in runs they stalled the wave's MFMAs: [4096,3072]x[3072,768] 208 us with the phases one after
 // another, 130 with fragments a step ahead, 112 dealt out evenly with eight waves).  Stage layout: per 16-k sub-step
@@ -692,7 +696,8 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
     constexpr int CB = BN * KB / NTHR >= 8 ? 8 : 4, NB = BN * KB / CB / NTHR;
     static_assert(NA * CA * NTHR == BM * KB && NB * CB * NTHR == BN * KB, "whole chunks");
     __shared__ __attribute__((aligned(1024))) char sm[2][STAGE];
-    __shared__ uint32_t amax[BM], bmax[BN];  // bits of the largest magnitude of each row and column
+    // of each row and column: the bits of its largest magnitude, and of its smallest but zero as (bits << 1) - 1
+    __shared__ uint32_t amax[BM], bmax[BN], amin[BM], bmin[BN];
     __shared__ ExpTable tab;
     if constexpr (GELU) exp_table_fill(tab);
     const int M = p.m, N = p.n;
@@ -705,8 +710,8 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
     const int nk = 2 * ((kr + 2 * KB - 1) / (2 * KB));                // steps, in pairs
     int64_t ao, bo, co;
     batch_offsets(p.batch_base + zb, p, &ao, &bo, &co);
-    for (int i = threadIdx.x; i < BM; i += blockDim.x) amax[i] = 0;
-    for (int i = threadIdx.x; i < BN; i += blockDim.x) bmax[i] = 0;
+    for (int i = threadIdx.x; i < BM; i += blockDim.x) amax[i] = 0, amin[i] = ~0u;
+    for (int i = threadIdx.x; i < BN; i += blockDim.x) bmax[i] = 0, bmin[i] = ~0u;
 
     // this thread's chunks: A chunk h is CA floats along K of one row (byte offset aoff, LDS offset ad); B chunk h is
     // CB k of one column (b by columns: as A's)
@@ -799,10 +804,11 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
     // instruction (or two) per pair, so that neighbouring instructions are independent
     constexpr int PA = NA * CA / 2, PB = NB * CB / 2, PT = PA + PB, U = (PT + 3) / 4, SEGS = 12 * U;
     float mxa[NA], mxb[NB];
+    uint32_t mna[NA], mnb[NB];
 #pragma unroll
-    for (int h = 0; h < NA; h++) mxa[h] = 0.f;
+    for (int h = 0; h < NA; h++) mxa[h] = 0.f, mna[h] = ~0u;
 #pragma unroll
-    for (int h = 0; h < NB; h++) mxb[h] = 0.f;
+    for (int h = 0; h < NB; h++) mxb[h] = 0.f, mnb[h] = ~0u;
     float res[8];
     uint32_t hi[8], pk[3][PT];
     // segment ic of the split of step kt's elements in s into stage ws; then loads step kl into s
@@ -826,7 +832,11 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
             if constexpr (sg == 1 || sg == 6) hi[2 * q] = pk[sg / 6][pr] << 16;
             if constexpr (sg == 2 || sg == 7) hi[2 * q + 1] = pk[sg / 6][pr] & 0xffff0000u;
             if constexpr (sg == 3) res[2 * q] = x[0] - __builtin_bit_cast(float, hi[2 * q]);
-            if constexpr (sg == 4) res[2 * q + 1] = x[1] - __builtin_bit_cast(float, hi[2 * q + 1]);
+            if constexpr (sg == 4) {
+                res[2 * q + 1] = x[1] - __builtin_bit_cast(float, hi[2 * q + 1]);
+                uint32_t &m = isA ? mna[isA ? h : 0] : mnb[isA ? 0 : h];
+                m = min(min((__builtin_bit_cast(uint32_t, x[0]) << 1) - 1u, (__builtin_bit_cast(uint32_t, x[1]) << 1) - 1u), m);
+            }
             if constexpr (sg == 5) {
                 pk[1][pr] = bf16_pair(res[2 * q], res[2 * q + 1]);
                 float &m = isA ? mxa[isA ? h : 0] : mxb[isA ? 0 : h];
@@ -854,12 +864,18 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
         });
     };
 
-    // the largest operand of each row and column
+    // the largest and the smallest operand of each row and column
     auto store_max = [&]() {
 #pragma unroll
-        for (int h = 0; h < NA; h++) atomicMax(&amax[ar[h]], __builtin_bit_cast(uint32_t, mxa[h]));
+        for (int h = 0; h < NA; h++) {
+            atomicMax(&amax[ar[h]], __builtin_bit_cast(uint32_t, mxa[h]));
+            atomicMin(&amin[ar[h]], mna[h]);
+        }
 #pragma unroll
-        for (int h = 0; h < NB; h++) atomicMax(&bmax[bc[h]], __builtin_bit_cast(uint32_t, mxb[h]));
+        for (int h = 0; h < NB; h++) {
+            atomicMax(&bmax[bc[h]], __builtin_bit_cast(uint32_t, mxb[h]));
+            atomicMin(&bmin[bc[h]], mnb[h]);
+        }
     };
     // parts of steps 0 and 1 into their stages, steps 2 and 3 loading
     Set s0, s1;
@@ -941,20 +957,35 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < MT; i++) {
+        constexpr uint32_t kLossy = ((127u - 109u) << 24) - 1u, kUnder = ((127u - 120u) << 24) - 1u;
         const float ra = __builtin_bit_cast(float, amax[wr + 32 * i + (l & 31)]);
+        const bool la = amin[wr + 32 * i + (l & 31)] < kLossy;
 #pragma unroll
         for (int j = 0; j < NT; j++) {
+            // whether the tile can hold such a result: one is not finite or nonzero below 2^-120, a row or column
+            // holds a value below 2^-109 or none of 2^-60 (lane l: row and column l % 32)
+            float top = 0.f;
+            uint32_t low = ~0u;
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+                const float v0 = acc[i][j][r], v1 = acc[i][j][r + 1];
+                top = __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(v0), fabsf(v1)), top);
+                low = min(min((__builtin_bit_cast(uint32_t, v0) << 1) - 1u, (__builtin_bit_cast(uint32_t, v1) << 1) - 1u), low);
+            }
+            const uint32_t lc = bmin[wc + 32 * j + (l & 31)];
+            const float c0 = __builtin_bit_cast(float, bmax[wc + 32 * j + (l & 31)]);
+            const bool odd = !(top < __builtin_inff()) || low < kUnder || la || lc < kLossy ||
+                             (ra != 0.f && ra < 0x1p-60f) || (c0 != 0.f && c0 < 0x1p-60f);
+            if (!__any(odd)) continue;
             uint32_t again = 0;
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                const float cb = __builtin_bit_cast(float, bmax[wc + 32 * j + 8 * (r / 4) + 4 * (l / 32) + r % 4]);
-                const float v = fabsf(acc[i][j][r]);
-                const bool ok = v >= fmaxf(ra, cb) * 0x1p-90f && v < __builtin_inff();
-                again |= (ok || ra == 0.f || cb == 0.f) ? 0u : 1u << r;
+                const int c = wc + 32 * j + 8 * (r / 4) + 4 * (l / 32) + r % 4;
+                const float cb = __builtin_bit_cast(float, bmax[c]), v = fabsf(acc[i][j][r]);
+                const bool lossy = v < fmaxf(la ? cb : 0.f, bmin[c] < kLossy ? ra : 0.f) * 0x1p-96f;
+                const bool under = v < 0x1p-120f && (v != 0.f || ra * cb < 0x1p-120f);
+                again |= (ra != 0.f && cb != 0.f && (lossy || under)) || !(v < __builtin_inff()) ? 1u << r : 0u;
             }
-            // (a zero row times an infinite or NaN column is not finite)
-#pragma unroll
-            for (int r = 0; r < 16; r++) again |= fabsf(acc[i][j][r]) < __builtin_inff() ? 0u : 1u << r;
             if (__any(again != 0)) {
                 const v16f x = f32_tile<BT>(A + ao, B + bo, M, N, p.lda, p.ldb, row0 + wr + 32 * i, col0 + wc + 32 * j,
                                             kbeg, kbeg + kr, l);

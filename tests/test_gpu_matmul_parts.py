@@ -4,9 +4,12 @@ the bf16 matrix unit (lx_matmul.hip, k_matmul_f32_b3).
 Bar: every part product is exact and each of a step's six MFMAs rounds its accumulation once, so a dot product of K
 terms is within (6 ceil(K / 16) + 1) 2^-24 sum_j |a_j b_j| of the exact one (the part products left out weigh 2^-25),
 and within the MatMul bar of 1e-5 sum_j |a_j b_j|."""
+import time
+
 import numpy as np
 import pytest
 
+import onnx_amd
 from onnx_amd import DeviceTensor, HipExecutionProvider as HIP, OpStatus
 
 pytestmark = pytest.mark.gpu
@@ -81,6 +84,38 @@ def test_parts_of_extreme_values(hip, m, k, n, kind):
         check(a[rows], b[:, cols], got[np.ix_(rows, cols)])
         return
     check(a, b)
+
+
+@pytest.mark.parametrize("m,k,n", [(4096, 768, 768), (788, 768, 768), (1100, 384, 1000)])
+def test_parts_time_does_not_depend_on_zeros(hip, m, k, n):
+    """Exactly zero results of nonzero rows and columns (integers, sparse operands, a selection) and small values need
+    no second run on the fp32 MFMA (which takes 3.4 to 5.5 times as long): the time of normal data, and integer
+    products are exact."""
+    rng = np.random.default_rng(17)
+    normal = [rng.standard_normal(s).astype(np.float32) for s in ((m, k), (k, n))]
+    small = [rng.integers(-8, 9, s).astype(np.float32) for s in ((m, k), (k, n))]
+    signs = [rng.integers(-1, 2, s).astype(np.float32) for s in ((m, k), (k, n))]
+    one = np.zeros((m, k), np.float32)
+    one[np.arange(m), rng.integers(0, k, m)] = 1
+    half = (normal[1] * (rng.random((k, n)) < 0.5)).astype(np.float32)
+    for a, b in (small, signs, [one, half]):
+        assert np.array_equal(mm(a, b), a.astype(np.float64) @ b.astype(np.float64))
+    y = DeviceTensor.empty((m, n), np.float32)
+    calls = {}
+    for name, (a, b) in {"normal": normal, "small": small, "signs": signs, "selected": (one, half),
+                         "tiny": (normal[0], (normal[1] * 1e-24).astype(np.float32))}.items():
+        calls[name] = (dev(a), dev(b))
+    best = dict.fromkeys(calls, 1e9)
+    for _ in range(5):
+        for name, (a, b) in calls.items():
+            HIP.MatMul(a, b, out=y)
+            onnx_amd.synchronize()
+            t = time.perf_counter()
+            for _ in range(50):
+                HIP.MatMul(a, b, out=y)
+            onnx_amd.synchronize()
+            best[name] = min(best[name], time.perf_counter() - t)
+    assert max(best.values()) < 2 * best["normal"], best
 
 
 def test_parts_results_do_not_depend_on_the_tile(hip):
