@@ -614,12 +614,17 @@ static void launch_f32_dl(const float *a, const float *b, float *c, const MatMul
 // x = p1 + p2 + p3 with p1 = bf16(x), p2 = bf16(x - p1), p3 = bf16(x - p1 - p2): three 8-bit significands hold all 24
 // bits of a float32, so the parts of a value of 2^-109 or more are exact.  A product is the six part products of
 // weight 2^-16 or more,
-//   a3 b1 + a1 b3 + a2 b2 + a2 b1 + a1 b2 + a1 b1
+//   (a3 b1 + a1 b3 + a2 b2 + a2 b1 + a1 b2) + a1 b1
 // (the three left out weigh 2^-25 |a b| at most), each exact in the MFMA and accumulated in float32: per step of 16
-// six v_mfma_f32_32x32x16_bf16 of 32 cycles, where v_mfma_f32_32x32x2f32 takes eight of 64.  Against 64 bits, normal
-// data, the relative error is below the fp32 MFMA's at every K: 1.6e-7 against 2.0e-7 (K 128), 2.9e-7 / 3.5e-7 (384),
-// 4.2e-7 / 5.0e-7 (768), 8.6e-7 / 1.0e-6 (3072), the small part products first as above (largest first: 1.8e-7 at
-// 128).  Shorter ranges stay on the fp32 MFMA: they are bound by launches and loads ([667,384]x[384,384] in ranges of
+// six v_mfma_f32_32x32x16_bf16 of 32 cycles, where v_mfma_f32_32x32x2f32 takes eight of 64.  The five small ones have
+// an accumulator of their own, added to the sum of the a1 b1 at the end: those have 16 significant bits, so that sum
+// hardly rounds, and the others round at 2^-8 of its size.  In one accumulator every MFMA rounded at full size, up to
+// twice as far off as a float32 chain where operands hold zeros (the chain does not round on a zero).  Relative error
+// against 64 bits, the fp32 MFMA's in brackets: normal data K 384 1.1e-7 (3.5e-7), 768 1.6e-7 (5.0e-7), 3072 3.4e-7
+// (9.9e-7); left operand 10% dense 4.6e-8 (1.1e-7), 6.1e-8 (1.6e-7), 1.2e-7 (3.2e-7), 2% dense 3.0e-8 (5.5e-8), 3.4e-8
+// (7.5e-8), 5.7e-8 (1.4e-7).  Only rows of a single nonzero product are off a little more, 2.60e-8 (2.53e-8, the
+// correctly rounded product), by the part products left out (none where one factor has 8 bits or fewer: a selection).
+// Shorter ranges stay on the fp32 MFMA: they are bound by launches and loads ([667,384]x[384,384] in ranges of
 // 128 ran slower in parts).  The choice is by the length of the K range alone, so that a product is the same bits in every tile, fused or not, folded or not.
 //
 // What the parts cannot hold goes to the fp32 MFMA, element by element: a result that is not finite (a value that is
@@ -916,13 +921,13 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
         if constexpr (z < MT) f.a[u][pa][z] = *(const v8bf *)(rs + u * SUB + pa * AP + fa + z * 512);
         else f.b[u][pb][z - MT] = *(const v8bf *)(rs + u * SUB + pb * BP + fb + (z - MT) * 512);
     };
-    v16f acc[MT][NT];
+    v16f acc[MT][NT], lo[MT][NT];  // the sums of a1 b1 and of the small part products
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
         for (int j = 0; j < NT; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+            for (int r = 0; r < 16; r++) acc[i][j][r] = lo[i][j][r] = 0.f;
     constexpr int G = 6 * MT * NT * KS, GD = G * 5 / 6;  // MFMAs per step; the other work follows the first GD of them
     auto step = [&](int kt, Set &s, const Frag &cur, Frag &nxt) {
         const char *rs = sm[(kt + 1) & 1];
@@ -932,7 +937,8 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
             constexpr int g = decltype(gc)::value, u = g / (6 * MT * NT), o = g % (6 * MT * NT), pr = o / (MT * NT);
             constexpr int i = o % (MT * NT) / NT, j = o % NT;
             constexpr int pa = pr == 0 ? 2 : pr == 1 || pr >= 4 ? 0 : 1, pb = pr == 1 ? 2 : pr == 2 || pr == 4 ? 1 : 0;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.b[u][pb][j], cur.a[u][pa][i], acc[i][j], 0, 0, 0);
+            v16f &sum = pr == 5 ? acc[i][j] : lo[i][j];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.b[u][pb][j], cur.a[u][pa][i], sum, 0, 0, 0);
             static_for<(g < GD ? g * R / GD : R), (g < GD ? (g + 1) * R / GD : R)>([&](auto c) { read_frag(c, rs, nxt); });
             if constexpr (PW == 0)
                 static_for<(g < GD ? g * SEGS / GD : SEGS), (g < GD ? (g + 1) * SEGS / GD : SEGS)>(
@@ -963,9 +969,12 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
 #pragma unroll
         for (int j = 0; j < NT; j++) {
             // whether the tile can hold such a result: one is not finite or nonzero below 2^-120, a row or column
-            // holds a value below 2^-109 or none of 2^-60 (lane l: row and column l % 32)
+            // holds a value below 2^-109, or the largest of a row and of a column multiply to less than 2^-120 (lane l:
+            // row and column l % 32)
             float top = 0.f;
             uint32_t low = ~0u;
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = acc[i][j][r] + lo[i][j][r];
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
                 const float v0 = acc[i][j][r], v1 = acc[i][j][r + 1];
@@ -974,9 +983,12 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
             }
             const uint32_t lc = bmin[wc + 32 * j + (l & 31)];
             const float c0 = __builtin_bit_cast(float, bmax[wc + 32 * j + (l & 31)]);
-            const bool odd = !(top < __builtin_inff()) || low < kUnder || la || lc < kLossy ||
-                             (ra != 0.f && ra < 0x1p-60f) || (c0 != 0.f && c0 < 0x1p-60f);
-            if (!__any(odd)) continue;
+            if (!__any(!(top < __builtin_inff()) || low < kUnder || la || lc < kLossy)) {
+                if (!__any((ra != 0.f && ra < 0x1p-60f) || (c0 != 0.f && c0 < 0x1p-60f))) continue;
+                float rm = ra != 0.f ? ra : __builtin_inff(), cm = c0 != 0.f ? c0 : __builtin_inff();
+                for (int o = 1; o < 32; o *= 2) rm = fminf(rm, __shfl_xor(rm, o)), cm = fminf(cm, __shfl_xor(cm, o));
+                if (!__any(rm * cm < 0x1p-120f)) continue;
+            }
             uint32_t again = 0;
 #pragma unroll
             for (int r = 0; r < 16; r++) {
@@ -1020,17 +1032,18 @@ static bool f32_b3(const MatMulArgs &p, int kr) {
     return kr >= kB3LoneK || blocks > 256;
 }
 
-// The block tile: the least estimated time.  A tile's step of 16 k takes `lone` us when its block has a CU to itself
-// and `full` us per block with r of them on a CU, measured over [4096, 384..3072] x [.., 384..3072], [788, ..] and
-// 2048^3: rounds of r blocks, then the rest.  64x64 with loading waves (12 waves: one block per CU) only up to 256
-// tiles.
+// The block tile: the least estimated time.  A block takes `fixed` us (first stage, check, stores) and per step of 16 k
+// `lone` us when it has a CU to itself, `full` us per block in a launch of several blocks per CU (r of them at once, else
+// one after another): rounds of r blocks, then the rest.  Fitted to [4096, 384..3072] x [.., 384..3072], [788, ..],
+// 1024^3 to 2048^3 and 12 batches of 384^3 and 512^3, where the tile it picks is the fastest of the four or within 4%.
 static int b3_tile(const MatMulArgs &p, bool only_general) {
     struct B3Tile {
         int bm, bn, r;
-        double lone, full;
+        double fixed, lone, full;
     };
-    static const B3Tile cand[] = {{128, 128, 2, 0.57, 0.72}, {128, 64, 2, 0.40, 0.50}, {64, 64, 3, 0.25, 0.25},
-                                  {64, 64, 1, 0.215, 0.39}};
+    static const B3Tile cand[] = {{128, 128, 1, 2.9, 0.58, 0.62}, {128, 64, 1, 1.8, 0.35, 0.44},
+                                  {64, 64, 3, 1.5, 0.27, 0.25}, {64, 64, 1, 1.0, 0.21, 0.28}};
+    const double steps = (double)((p.k + 15) / 16);
     int best = 0;
     double cost = 0;
     for (int i = 0; i < 4; i++) {
@@ -1038,7 +1051,9 @@ static int b3_tile(const MatMulArgs &p, bool only_general) {
         const B3Tile &c = cand[i];
         const int64_t tiles = (int64_t)((p.m + c.bm - 1) / c.bm) * ((p.n + c.bn - 1) / c.bn) * p.batch;
         const int64_t per_cu = (tiles + 255) / 256, rounds = per_cu / c.r, rest = per_cu - rounds * c.r;
-        const double t = per_cu == 1 ? c.lone : rounds * c.r * c.full + (rest > 1 ? rest * c.full : rest * c.lone);
+        const double t = per_cu == 1 ? c.fixed + steps * c.lone
+                                     : rounds * (c.fixed + steps * c.r * c.full) +
+                                           (rest ? c.fixed + steps * (rest > 1 ? rest * c.full : c.lone) : 0);
         if (i == 0 || t < cost) {
             best = i;
             cost = t;
@@ -1068,23 +1083,23 @@ static void launch_f32_b3(const float *a, const float *b, float *c, const MatMul
     const bool whole = va && p.k % 64 == 0;  // whole step pairs of every tile
     const int tile = b3_tile(p, p.bt || !whole);
     if (p.bt) {
-        if (whole && tile == 0) b3_launch<128, 128, 2, 4, 0, 1, 4, true, false, true>(a, b, c, p, vec, s);
+        if (whole && tile == 0) b3_launch<128, 128, 2, 4, 0, 1, 2, true, false, true>(a, b, c, p, vec, s);
         else if (whole) b3_launch<64, 64, 2, 2, 0, 2, 3, true, false, true>(a, b, c, p, vec, s);
         else b3_launch<64, 64, 2, 2, 0, 2, 2, false, true, true>(a, b, c, p, vec, s);
         return;
     }
     if (!va) {  // unaligned rows: scalar loads
-        if (tile == 0) b3_launch<128, 128, 2, 4, 0, 1, 4, false, true, false>(a, b, c, p, vec, s);
+        if (tile == 0) b3_launch<128, 128, 2, 4, 0, 1, 2, false, true, false>(a, b, c, p, vec, s);
         else b3_launch<64, 64, 2, 2, 0, 2, 2, false, true, false>(a, b, c, p, vec, s);
         return;
     }
     if (!whole) {
-        if (tile == 0) b3_launch<128, 128, 2, 4, 0, 1, 4, true, true, false>(a, b, c, p, vec, s);
+        if (tile == 0) b3_launch<128, 128, 2, 4, 0, 1, 2, true, true, false>(a, b, c, p, vec, s);
         else b3_launch<64, 64, 2, 2, 0, 2, 2, true, true, false>(a, b, c, p, vec, s);
         return;
     }
     switch (tile) {
-    case 0: b3_launch<128, 128, 2, 4, 0, 1, 4, true, false, false>(a, b, c, p, vec, s); break;
+    case 0: b3_launch<128, 128, 2, 4, 0, 1, 2, true, false, false>(a, b, c, p, vec, s); break;
     case 1: b3_launch<128, 64, 4, 2, 0, 2, 2, true, false, false>(a, b, c, p, vec, s); break;
     case 2: b3_launch<64, 64, 2, 2, 0, 2, 3, true, false, false>(a, b, c, p, vec, s); break;
     default: b3_launch<64, 64, 2, 2, 8, 2, 3, true, false, false>(a, b, c, p, vec, s); break;

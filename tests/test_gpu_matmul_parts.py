@@ -86,6 +86,38 @@ def test_parts_of_extreme_values(hip, m, k, n, kind):
     check(a, b)
 
 
+def float32_chain(a, b):
+    """The products one after another in float32, each exact before it is added (a chain of fused multiply-adds, which
+    v_mfma_f32_32x32x2f32 is): float64 holds a product's 48 bits and adds it with an error far below a float32's."""
+    acc = np.zeros((a.shape[0], b.shape[1]), np.float32)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    for j in range(a.shape[1]):
+        acc = (acc + a[:, j:j + 1] * b[j]).astype(np.float32)
+    return acc
+
+
+# 128x64, 64x64, 128x128 tiles, loading waves, a split product, scalar loads with a tail
+@pytest.mark.parametrize("m,k,n", [(1100, 384, 960), (600, 516, 516), (788, 768, 2500), (700, 768, 768), (8, 2048, 4096),
+                                   (1090, 333, 1000)])
+@pytest.mark.parametrize("dense", [1.0, 0.5, 0.1, 0.02, "both", "positive", "small"])
+def test_parts_error_is_no_larger_than_a_float32_chain(hip, m, k, n, dense):
+    """Against 64 bits, dense and sparse operands (a float32 chain does not round on a zero)."""
+    rng = np.random.default_rng(19)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    if dense == "positive":
+        a, b = np.abs(a), np.abs(b)
+    elif dense == "small":  # small part products of subnormal size, results just above where they run again
+        a, b = a * np.float32(2.0 ** -58), b * np.float32(2.0 ** -58)
+    elif dense == "both":
+        a, b = a * (rng.random(a.shape) < 0.1), b * (rng.random(b.shape) < 0.1)
+    else:
+        a *= rng.random(a.shape) < dense
+    got = mm(a.astype(np.float32), b.astype(np.float32)).astype(np.float64)
+    rows, cols = slice(0, 64), slice(0, min(n, 512))
+    exact, chain = a[rows].astype(np.float64) @ b[:, cols].astype(np.float64), float32_chain(a[rows], b[:, cols])
+    assert np.linalg.norm(got[rows, cols] - exact) <= np.linalg.norm(chain - exact)
+
+
 @pytest.mark.parametrize("m,k,n", [(4096, 768, 768), (788, 768, 768), (1100, 384, 1000)])
 def test_parts_time_does_not_depend_on_zeros(hip, m, k, n):
     """Exactly zero results of nonzero rows and columns (integers, sparse operands, a selection) and small values need
