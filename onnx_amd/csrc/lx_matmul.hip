@@ -1016,19 +1016,21 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
         mm_epilogue<MT, NT, false, GELU>(acc, C, p, co, row0 + wr, col0 + wc, l, tab);
 }
 
-constexpr int kB3MinK = 256, kB3LoneK = 512;
+constexpr int kB3MinK = 256, kB3LoneK = 512, kB3SplitK = 1024;
 // Whether a K range of kr goes to k_matmul_f32_b3: kB3MinK or more, N above 32 (a context product of 32-wide heads is
 // bound by its loads: [96,512,512]x[96,512,32] 24 us on the fp32 MFMA, 26 in parts), and strides whose offsets within
 // a tile and a step stay below 2^31 bytes (rows of up to 8 MB; longer ones keep the fp32 MFMA).  A range below kB3LoneK
 // whose blocks (of one matrix in a grouped launch, which has to give the bits of its single products) find a CU each
 // keeps the fp32 MFMA too: the parts' first stage and last check cost 1.2 us more than a block of so few steps gains
-// ([640,1536]x[1536,384] 14.9 against 13.2 us a call, six batches of 384^3 11.8 against 10.2; [1024,512]x[512,512],
-// the first on the other side, 11.3 against 11.2).
+// (six batches of 384^3 11.8 against 10.2 us; [1024,512]x[512,512], the first on the other side, 11.0 in both).  The
+// ranges of a split product, at most one block per CU and mostly of few rows, keep it up to kB3SplitK: there the parts'
+// 4-byte loads of B count too (ranges of 512: [60,2560]x[2560,4096] 18.0 us in parts, 16.5; 768: [256,3072]x[3072,768]
+// 18.9, 18.3; 1024: [384,3072]x[3072,768] 22.6, 22.5; 1536: [640,3072]x[3072,640] 29.3, 30.1).
 static bool f32_b3(const MatMulArgs &p, int kr) {
     const int64_t lim = (int64_t)1 << 21;
     if (kr < kB3MinK || p.n <= 32 || p.lda > lim || p.ldb > lim || p.k > (1 << 24)) return false;
-    const int64_t blocks = (((int64_t)p.m + 63) / 64) * (((int64_t)p.n + 63) / 64) * (p.k / kr) *
-                           (p.split_per_matrix ? 1 : p.batch);
+    if (kr < p.k) return kr > kB3SplitK;
+    const int64_t blocks = (((int64_t)p.m + 63) / 64) * (((int64_t)p.n + 63) / 64) * (p.split_per_matrix ? 1 : p.batch);
     return kr >= kB3LoneK || blocks > 256;
 }
 

@@ -97,7 +97,7 @@ def float32_chain(a, b):
 
 
 # 128x64, 64x64, 128x128 tiles, loading waves, a split product, scalar loads with a tail
-@pytest.mark.parametrize("m,k,n", [(1100, 384, 960), (600, 516, 516), (788, 768, 2500), (700, 768, 768), (8, 2048, 4096),
+@pytest.mark.parametrize("m,k,n", [(1100, 384, 960), (600, 516, 516), (788, 768, 2500), (700, 768, 768), (8, 4096, 4096),
                                    (1090, 333, 1000)])
 @pytest.mark.parametrize("dense", [1.0, 0.5, 0.1, 0.02, "both", "positive", "small"])
 def test_parts_error_is_no_larger_than_a_float32_chain(hip, m, k, n, dense):
@@ -116,6 +116,22 @@ def test_parts_error_is_no_larger_than_a_float32_chain(hip, m, k, n, dense):
     rows, cols = slice(0, 64), slice(0, min(n, 512))
     exact, chain = a[rows].astype(np.float64) @ b[:, cols].astype(np.float64), float32_chain(a[rows], b[:, cols])
     assert np.linalg.norm(got[rows, cols] - exact) <= np.linalg.norm(chain - exact)
+
+
+@pytest.mark.parametrize("m,k,n,r", [(60, 2560, 4096, 4), (256, 3072, 768, 4), (384, 3072, 768, 3)])
+def test_short_ranges_of_a_split_product_keep_float32(hip, m, k, n, r):
+    """Ranges of up to 1024 run on the fp32 MFMA, where they are faster: each partial product is the bits of a float32
+    chain of steps of 16, k = j and then k = 8 + j of each (j = 0..7), and the partials are added in order."""
+    rng = np.random.default_rng(23)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    order = np.arange(k).reshape(-1, 2, 8).transpose(0, 2, 1).reshape(-1)
+    got, cols = mm(a, b), slice(n - 64, n)
+    ref = np.zeros((8, 64), np.float32)
+    for i in range(r):
+        o = order[i * (k // r):(i + 1) * (k // r)]
+        part = float32_chain(a[:8, o], b[o, cols])
+        ref = part if i == 0 else ref + part
+    assert np.array_equal(got[:8, cols], ref)
 
 
 @pytest.mark.parametrize("m,k,n", [(4096, 768, 768), (788, 768, 768), (1100, 384, 1000)])
