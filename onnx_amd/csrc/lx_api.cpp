@@ -1970,6 +1970,10 @@ int api_matmul_permuted(const lx_tensor *A, const int *a_perm, const lx_tensor *
         return true;
     };
     if (!permute(x, a_perm, false) || !permute(y, b_perm, true)) return LX_ERR_NOT_SUPPORTED;
+    // rows of a view further apart than the dense tensor's could move the product to another unit, and its last bits
+    for (const MView *v : {&x, &y})
+        for (int i = std::max(0, v->rank - 2); i < v->rank; i++)
+            if (v->dims[i] > 1 && v->str[i] > kMatMulPartsRow) return LX_ERR_NOT_SUPPORTED;
     std::vector<void *> temps;
     MatMulOpts o;
     o.yperm = y_perm;

@@ -220,6 +220,8 @@ struct MatMulArgs {
 };
 // Bytes of partial products launch_matmul needs in MatMulArgs::part for these operands (0: no split).
 constexpr int64_t kMatMulSplitBatch = 16;
+// Longest row stride (elements) of a Float operand whose products may run in bf16 parts.
+constexpr int64_t kMatMulPartsRow = (int64_t)1 << 21;
 int64_t matmul_part_bytes(int dtype, const void *a, const void *b, const void *c, const MatMulArgs &p);
 hipError_t launch_matmul(int dtype, const void *a, const void *b, void *c, const MatMulArgs &p, hipStream_t s);
 // A split Float product (its epilogue included, no GELU) whose rows of n (a multiple of 4, 256 to 4096) are then

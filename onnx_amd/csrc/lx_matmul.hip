@@ -625,7 +625,8 @@ static void launch_f32_dl(const float *a, const float *b, float *c, const MatMul
 // (7.5e-8), 5.7e-8 (1.4e-7).  Only rows of a single nonzero product are off a little more, 2.60e-8 (2.53e-8, the
 // correctly rounded product), by the part products left out (none where one factor has 8 bits or fewer: a selection).
 // Shorter ranges stay on the fp32 MFMA: they are bound by launches and loads ([667,384]x[384,384] in ranges of
-// 128 ran slower in parts).  The choice is by the length of the K range alone, so that a product is the same bits in every tile, fused or not, folded or not.
+// 128 ran slower in parts).  f32_b3 chooses by the K range, N, the row strides and f32_tiles, none of which depends on the
+// block tile or on what is fused or folded: a product is the same bits in all of these forms.
 //
 // What the parts cannot hold goes to the fp32 MFMA, element by element: a result that is not finite (a value that is
 // not, or rounds to an infinite bf16); a result smaller than 2^-96 of its column's largest operand where its row holds
@@ -1016,22 +1017,36 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
         mm_epilogue<MT, NT, false, GELU>(acc, C, p, co, row0 + wr, col0 + wc, l, tab);
 }
 
+// 64x64 tiles of a float product, the count that its split and its unit go by: of the whole call, not of a launch's share
+// of a large batch; of one matrix in a grouped launch, which has to give the bits of its single products; and of the
+// rows of the whole batch where every matrix of it meets one right operand, whether the call could fold them into one
+// product (dense rows) or not (a transposed view, a bias row per batch), so that both are the same bits.
+static int64_t f32_tiles(const MatMulArgs &p) {
+    const int64_t cols = ((int64_t)p.n + 63) / 64;
+    if (p.split_per_matrix) return ((int64_t)p.m + 63) / 64 * cols;
+    int64_t batch = 1;
+    bool shared = true;
+    for (int d = 0; d < p.nbatch; d++) {
+        batch *= p.bdims[d];
+        shared = shared && (p.bdims[d] == 1 || p.b_bstr[d] == 0);
+    }
+    return shared ? (p.m * batch + 63) / 64 * cols : ((int64_t)p.m + 63) / 64 * cols * batch;
+}
+
 constexpr int kB3MinK = 256, kB3LoneK = 512, kB3SplitK = 1024;
 // Whether a K range of kr goes to k_matmul_f32_b3: kB3MinK or more, N above 32 (a context product of 32-wide heads is
 // bound by its loads: [96,512,512]x[96,512,32] 24 us on the fp32 MFMA, 26 in parts), and strides whose offsets within
 // a tile and a step stay below 2^31 bytes (rows of up to 8 MB; longer ones keep the fp32 MFMA).  A range below kB3LoneK
-// whose blocks (of one matrix in a grouped launch, which has to give the bits of its single products) find a CU each
-// keeps the fp32 MFMA too: the parts' first stage and last check cost 1.2 us more than a block of so few steps gains
+// whose 64x64 tiles (f32_tiles) find a CU each keeps the fp32 MFMA too: the parts' first stage and last check cost 1.2 us more than a block of so few steps gains
 // (six batches of 384^3 11.8 against 10.2 us; [1024,512]x[512,512], the first on the other side, 11.0 in both).  The
 // ranges of a split product, at most one block per CU and mostly of few rows, keep it up to kB3SplitK: there the parts'
 // 4-byte loads of B count too (ranges of 512: [60,2560]x[2560,4096] 18.0 us in parts, 16.5; 768: [256,3072]x[3072,768]
 // 18.9, 18.3; 1024: [384,3072]x[3072,768] 22.6, 22.5; 1536: [640,3072]x[3072,640] 29.3, 30.1).
 static bool f32_b3(const MatMulArgs &p, int kr) {
-    const int64_t lim = (int64_t)1 << 21;
+    const int64_t lim = kMatMulPartsRow;
     if (kr < kB3MinK || p.n <= 32 || p.lda > lim || p.ldb > lim || p.k > (1 << 24)) return false;
     if (kr < p.k) return kr > kB3SplitK;
-    const int64_t blocks = (((int64_t)p.m + 63) / 64) * (((int64_t)p.n + 63) / 64) * (p.split_per_matrix ? 1 : p.batch);
-    return kr >= kB3LoneK || blocks > 256;
+    return kr >= kB3LoneK || f32_tiles(p) > 256;
 }
 
 // The block tile: the least estimated time.  A block takes `fixed` us (first stage, check, stores) and per step of 16 k
@@ -1684,17 +1699,15 @@ static bool f32_vec(const void *a, const void *b, const void *c, const MatMulArg
 }
 
 // K ranges of a float product on the direct-load kernel's terms (16-byte operands, K a multiple of 64): with
-// T tiles of 64x64 over the batch (ceil(m / 64) ceil(n / 64) per matrix), the most ranges, each a whole number
+// T tiles of 64x64 (f32_tiles), the most ranges, each a whole number
 // of passes of 64, that divide K / 64 into equal parts and keep T times the ranges within 256 blocks (one per
 // CU); 1 when T alone reaches 128 or K is a single pass.  A product of few tiles otherwise leaves
 // most CUs idle while its blocks each walk the whole of K ([8,1536] x [1536,384]: 6 blocks).  With
-// split_per_matrix, T counts one matrix's tiles (and a batch above kMatMulSplitBatch does not split), so
-// that each matrix of a grouped launch splits as it does alone.
+// split_per_matrix (T counts one matrix's tiles) a batch above kMatMulSplitBatch does not split.
 static int f32_split(const MatMulArgs &p, bool vec) {
     if (!vec || p.k % 64 != 0) return 1;
-    const int64_t per = (((int64_t)p.m + 63) / 64) * (((int64_t)p.n + 63) / 64);
     if (p.split_per_matrix && p.batch > kMatMulSplitBatch) return 1;
-    const int64_t tiles = p.split_per_matrix ? per : per * p.batch;
+    const int64_t tiles = f32_tiles(p);
     if (tiles >= 128) return 1;
     const int steps = p.k / 64;
     int best = 1;

@@ -200,3 +200,48 @@ def test_parts_of_a_right_operand_by_columns(hip, s, d):
         res.append(g.Output("y").to_numpy())
     assert np.array_equal(res[0].view(np.uint32), res[1].view(np.uint32))
     check(ins["q"].transpose(0, 2, 1, 3), ins["k"].transpose(0, 2, 3, 1), res[1])
+
+
+@pytest.mark.parametrize("b,m,k,n", [(192, 8, 384, 384), (64, 8, 384, 384), (600, 4, 320, 512), (40, 70, 1536, 96)])
+@pytest.mark.parametrize("side", ["left", "result"])
+def test_a_shared_right_operand_is_the_same_bits_folded_or_not(hip, b, m, k, n, side):
+    """A product whose left matrices all meet one right matrix runs as one product of their rows where these are
+    dense, and batch by batch where the Transpose before or after it is folded in: both split K and choose their unit
+    by the rows of the whole batch (three ranges, the fp32 MFMA, parts, ranges of a split product)."""
+    import onnx_writer as W
+    from onnx_amd.graph import Model
+    rng = np.random.default_rng(29)
+    x = rng.standard_normal((m, b, k) if side == "left" else (b, m, k)).astype(np.float32)
+    w = rng.standard_normal((k, n)).astype(np.float32)
+    nodes = ([W.node("Transpose", ["x"], ["t"], "t", perm=[1, 0, 2]), W.node("MatMul", ["t", "w"], ["y"], "mm")]
+             if side == "left" else
+             [W.node("MatMul", ["x", "w"], ["t"], "mm"), W.node("Transpose", ["t"], ["y"], "t", perm=[1, 0, 2])])
+    res = []
+    for fuse in (False, True):
+        g = Model.Load(W.model(nodes, [("x", np.float32, x.shape)], [("y", np.float32, ())], [("w", w)]))
+        if fuse:
+            assert g.Fuse() == 1 and [v.Op for v in g.Nodes] == ["MatMulPermuted"]
+        assert g.Execute({"x": dev(x)}), g.LastError
+        res.append(g.Output("y").to_numpy())
+    assert np.array_equal(res[0].view(np.uint32), res[1].view(np.uint32))
+    check(x.swapaxes(0, 1) if side == "left" else x, w, res[0] if side == "left" else res[0].swapaxes(0, 1))
+
+
+@pytest.mark.parametrize("b,m,k,n", [(192, 8, 384, 384), (600, 4, 320, 512)])
+def test_a_bias_row_per_batch_keeps_the_products_bits(hip, b, m, k, n):
+    rng = np.random.default_rng(31)
+    x, w = rng.standard_normal((b, m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    bias = rng.standard_normal((b, 1, n)).astype(np.float32)
+    r = HIP.MatMulAdd(dev(x), dev(w), dev(bias))
+    assert r.Status == OpStatus.Success, r.Message
+    assert np.array_equal(r.Outputs[0].to_numpy(), mm(x, w) + bias)
+
+
+def test_a_large_batch_runs_on_one_unit(hip):
+    """Batches above 65535 run in several launches: the last, short one keeps the unit of the others."""
+    rng = np.random.default_rng(37)
+    a, b = rng.standard_normal((41, 1600, 1, 256)).astype(np.float32), rng.standard_normal((1600, 256, 33)).astype(np.float32)
+    a[40] = a[0]
+    got = mm(a, b)
+    assert np.array_equal(got[40], got[0])
+    check(a[0], b, got[0])
