@@ -70,7 +70,9 @@ int api_matmul_add_layernorm(const lx_tensor *A, const lx_tensor *W, const lx_te
 // MatMul of transpose(A, a_perm) and transpose(B, b_perm) (null: the tensor itself), its product stored as
 // transpose(product, y_perm) into Y (null: as it is), Float, each permutation keeping the last axis last: the
 // kernels read and write the transposed views through their strides, and the result is bit for bit the
-// Transpose nodes' and MatMul's.  LX_ERR_NOT_SUPPORTED (no message) for operands it does not take.
+// Transpose nodes' and MatMul's (but where a batch over one right matrix has fewer than 128 tiles of 64x64 as one
+// product of all its rows: the MatMul node runs that and splits K, the views keep the batch).  LX_ERR_NOT_SUPPORTED
+// (no message) for operands it does not take.
 int api_matmul_permuted(const lx_tensor *A, const int *a_perm, const lx_tensor *B, const int *b_perm,
                         const int *y_perm, lx_tensor *Y);
 // An attention head's scores transpose(Q, q_perm) x transpose(K, k_perm), their Softmax along the last axis

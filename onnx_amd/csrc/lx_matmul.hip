@@ -626,7 +626,7 @@ static void launch_f32_dl(const float *a, const float *b, float *c, const MatMul
 // correctly rounded product), by the part products left out (none where one factor has 8 bits or fewer: a selection).
 // Shorter ranges stay on the fp32 MFMA: they are bound by launches and loads ([667,384]x[384,384] in ranges of
 // 128 ran slower in parts).  f32_b3 chooses by the K range, N, the row strides and f32_tiles, none of which depends on the
-// block tile or on what is fused or folded: a product is the same bits in all of these forms.
+// block tile or on what is fused or folded: an unsplit product is the same bits in all of these forms.
 //
 // What the parts cannot hold goes to the fp32 MFMA, element by element: a result that is not finite (a value that is
 // not, or rounds to an infinite bf16); a result smaller than 2^-96 of its column's largest operand where its row holds
@@ -1017,20 +1017,19 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
         mm_epilogue<MT, NT, false, GELU>(acc, C, p, co, row0 + wr, col0 + wc, l, tab);
 }
 
-// 64x64 tiles of a float product, the count that its split and its unit go by: of the whole call, not of a launch's share
-// of a large batch; of one matrix in a grouped launch, which has to give the bits of its single products; and of the
-// rows of the whole batch where every matrix of it meets one right operand, whether the call could fold them into one
-// product (dense rows) or not (a transposed view, a bias row per batch), so that both are the same bits.
-static int64_t f32_tiles(const MatMulArgs &p) {
+// 64x64 tiles of a float product: of the whole call, not of a launch's share of a large batch, and of one matrix in a
+// grouped launch, which has to give the bits of its single products.  `fold`: of the rows of the whole batch where every
+// matrix of it meets one right operand, whether the call could fold them into one product (dense rows) or not (a
+// transposed view, a bias row per batch), so that both run on one unit.
+static int64_t f32_tiles(const MatMulArgs &p, bool fold) {
     const int64_t cols = ((int64_t)p.n + 63) / 64;
     if (p.split_per_matrix) return ((int64_t)p.m + 63) / 64 * cols;
     int64_t batch = 1;
-    bool shared = true;
     for (int d = 0; d < p.nbatch; d++) {
         batch *= p.bdims[d];
-        shared = shared && (p.bdims[d] == 1 || p.b_bstr[d] == 0);
+        fold = fold && (p.bdims[d] == 1 || p.b_bstr[d] == 0);
     }
-    return shared ? (p.m * batch + 63) / 64 * cols : ((int64_t)p.m + 63) / 64 * cols * batch;
+    return fold ? (p.m * batch + 63) / 64 * cols : ((int64_t)p.m + 63) / 64 * cols * batch;
 }
 
 constexpr int kB3MinK = 256, kB3LoneK = 512, kB3SplitK = 1024;
@@ -1046,7 +1045,7 @@ static bool f32_b3(const MatMulArgs &p, int kr) {
     const int64_t lim = kMatMulPartsRow;
     if (kr < kB3MinK || p.n <= 32 || p.lda > lim || p.ldb > lim || p.k > (1 << 24)) return false;
     if (kr < p.k) return kr > kB3SplitK;
-    return kr >= kB3LoneK || f32_tiles(p) > 256;
+    return kr >= kB3LoneK || f32_tiles(p, true) > 256;
 }
 
 // The block tile: the least estimated time.  A block takes `fixed` us (first stage, check, stores) and per step of 16 k
@@ -1699,7 +1698,7 @@ static bool f32_vec(const void *a, const void *b, const void *c, const MatMulArg
 }
 
 // K ranges of a float product on the direct-load kernel's terms (16-byte operands, K a multiple of 64): with
-// T tiles of 64x64 (f32_tiles), the most ranges, each a whole number
+// T tiles of 64x64 over the batch as it is launched (f32_tiles), the most ranges, each a whole number
 // of passes of 64, that divide K / 64 into equal parts and keep T times the ranges within 256 blocks (one per
 // CU); 1 when T alone reaches 128 or K is a single pass.  A product of few tiles otherwise leaves
 // most CUs idle while its blocks each walk the whole of K ([8,1536] x [1536,384]: 6 blocks).  With
@@ -1707,7 +1706,7 @@ static bool f32_vec(const void *a, const void *b, const void *c, const MatMulArg
 static int f32_split(const MatMulArgs &p, bool vec) {
     if (!vec || p.k % 64 != 0) return 1;
     if (p.split_per_matrix && p.batch > kMatMulSplitBatch) return 1;
-    const int64_t tiles = f32_tiles(p);
+    const int64_t tiles = f32_tiles(p, false);
     if (tiles >= 128) return 1;
     const int steps = p.k / 64;
     int best = 1;

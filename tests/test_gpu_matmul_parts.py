@@ -202,12 +202,12 @@ def test_parts_of_a_right_operand_by_columns(hip, s, d):
     check(ins["q"].transpose(0, 2, 1, 3), ins["k"].transpose(0, 2, 3, 1), res[1])
 
 
-@pytest.mark.parametrize("b,m,k,n", [(192, 8, 384, 384), (64, 8, 384, 384), (600, 4, 320, 512), (40, 70, 1536, 96)])
+@pytest.mark.parametrize("b,m,k,n", [(192, 8, 384, 384), (600, 4, 320, 512), (40, 220, 1536, 96)])
 @pytest.mark.parametrize("side", ["left", "result"])
 def test_a_shared_right_operand_is_the_same_bits_folded_or_not(hip, b, m, k, n, side):
     """A product whose left matrices all meet one right matrix runs as one product of their rows where these are
-    dense, and batch by batch where the Transpose before or after it is folded in: both split K and choose their unit
-    by the rows of the whole batch (three ranges, the fp32 MFMA, parts, ranges of a split product)."""
+    dense, and batch by batch where the Transpose before or after it is folded in: both choose their unit by the rows of
+    the whole batch (the fp32 MFMA, parts of a short and of a long K)."""
     import onnx_writer as W
     from onnx_amd.graph import Model
     rng = np.random.default_rng(29)
