@@ -1229,8 +1229,17 @@ __global__ __launch_bounds__(1024) void k_matmul_small(const float *__restrict__
 // right operand again from L2, and above a tile of 64 the ranges of a long K are no longer 64.  Blocks of eight rows
 // measured slower up to 64 rows (32 rows: 473 against 430 us for the 12-layer encoder).
 constexpr int kSmallM = 64;
-static bool f32_small(const MatMulArgs &p, int split) {
-    return split > 1 && split <= kSmallRanges && p.k / split == 64 && p.m <= kSmallM && !p.bt;
+static bool f32_small(const void *a, const void *b, const void *c, const MatMulArgs &p, int split) {
+    if (split <= 1 || split > kSmallRanges || p.k / split != 64 || p.m > kSmallM || p.bt) return false;
+    // a result over an operand: blocks still read what others have written (the two launches read both first)
+    int64_t ea = (int64_t)(p.m - 1) * p.lda + p.k, eb = (int64_t)(p.k - 1) * p.ldb + p.n, ec = (int64_t)(p.m - 1) * p.ldc + p.n;
+    for (int d = 0; d < p.nbatch; d++) {
+        ea += (p.bdims[d] - 1) * p.a_bstr[d];
+        eb += (p.bdims[d] - 1) * p.b_bstr[d];
+        ec += (p.bdims[d] - 1) * p.c_bstr[d];
+    }
+    const float *fa = (const float *)a, *fb = (const float *)b, *fc = (const float *)c;
+    return !(fc < fa + ea && fa < fc + ec) && !(fc < fb + eb && fb < fc + ec);
 }
 static void launch_f32_small(const float *a, const float *b, float *c, const MatMulArgs &p, hipStream_t s) {
     const dim3 g((p.n + kSmallC - 1) / kSmallC, (p.m + kSmallR - 1) / kSmallR, (unsigned)p.batch);
@@ -1743,7 +1752,7 @@ hipError_t launch_matmul_ln(const void *a, const void *b, void *y, const MatMulA
 int64_t matmul_part_bytes(int dtype, const void *a, const void *b, const void *c, const MatMulArgs &p) {
     if (dtype != kFloat || p.m == 0 || p.n == 0 || p.batch == 0) return 0;
     const int r = f32_split(p, f32_vec(a, b, c, p));
-    return r > 1 && !f32_small(p, r) ? (int64_t)r * p.batch * p.m * p.n * (int64_t)sizeof(float) : 0;
+    return r > 1 && !f32_small(a, b, c, p, r) ? (int64_t)r * p.batch * p.m * p.n * (int64_t)sizeof(float) : 0;
 }
 
 hipError_t launch_matmul(int dtype, const void *a, const void *b, void *c, const MatMulArgs &p0, hipStream_t s) {
@@ -1765,7 +1774,7 @@ hipError_t launch_matmul(int dtype, const void *a, const void *b, void *c, const
         const float *fa = (const float *)a, *fb = (const float *)b;
         float *fc = (float *)c;
         const int split = f32_split(p, vec);
-        if (f32_small(p, split)) {
+        if (f32_small(a, b, c, p, split)) {
             MatMulArgs q = p;
             q.split = split;
             launch_f32_small(fa, fb, fc, q, s);

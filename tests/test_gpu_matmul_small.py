@@ -70,3 +70,17 @@ def test_small_products_of_not_finite_values(hip):
     assert np.array_equal(np.isnan(ref), np.isnan(got))
     inf = np.isinf(ref)
     assert np.array_equal(inf, np.isinf(got)) and np.array_equal(ref[inf], got[inf])
+
+
+@pytest.mark.parametrize("m,n,batch", [(8, 384, 1), (64, 256, 1), (5, 192, 3)])
+def test_small_products_over_their_operands(hip, m, n, batch):
+    """A result stored over the left operand, or over the residual: the bits of a result of its own."""
+    rng = np.random.default_rng(8)
+    for _ in range(5):
+        a, b = (rng.standard_normal((batch, r, n)).astype(np.float32) for r in (m, n))
+        bias, ref = rng.standard_normal(n).astype(np.float32), out(HIP.MatMul(dev(a), dev(b)))
+        x, r = dev(a), dev(a)
+        same(out(HIP.MatMul(x, dev(b), out=x)), ref)
+        x = dev(a)
+        same(out(HIP.MatMulAdd(x, dev(b), dev(bias), x, out=x)), (ref + bias) + a)
+        same(out(HIP.MatMulAdd(dev(a), dev(b), dev(bias), r, out=r)), (ref + bias) + a)
