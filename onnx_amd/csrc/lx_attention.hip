@@ -6,8 +6,11 @@
 // wave per SIMD does not cover: [8,12,512,512] heads of 32 52 us with one wave per 32 rows, 46 with two in blocks of
 // 128 rows, 38 in blocks of 64, which spread evenly over the CUs.)  Products run
 // on the bf16 matrix unit with every operand in three bf16 parts, as k_matmul_f32_b3's (lx_matmul.hip): p1 = bf16(x),
-// p2 = bf16(x - p1), p3 = bf16(x - p1 - p2), six part products per product, the small ones first, accumulated in
-// float32.  Both products run transposed, so that nothing crosses lanes in between:
+// p2 = bf16(x - p1), p3 = bf16(x - p1 - p2), six part products per product, accumulated in float32: for the scores the
+// small ones of all D first, for the context in an accumulator of their own (in one, every MFMA rounded at the size of
+// the whole sum).  Against 64 bits, the three float32 nodes in brackets, [2,4,512,512] heads of 64: normal values
+// 1.5e-7 (3.5e-7), ReLU'd V 8.1e-8 (8.7e-8), a tenth of Q, K and V 7.1e-8 (9.8e-8), 3% of the keys 1.0e-7 (1.8e-7);
+// [2,4,197,197] 1.4e-7 (3.5e-7), 7.0e-8 (1.5e-7), 6.9e-8 (9.7e-8), 8.2e-8 (1.4e-7).  Both products run transposed, so that nothing crosses lanes in between:
 //   scores^T  = K Q^T  : lane l holds query l % 32 and keys 8 (r / 4) + 4 (l / 32) + r % 4 of the tile (r = 0..15);
 //   context^T = V^T P^T: r = 8 c + j is then the lane's k slot j of the 16 keys c, the order V's tile is stored in.
 // The Softmax is the running one: a reference m per row (the row's largest score so far; it follows a new largest
@@ -62,15 +65,16 @@ __device__ __forceinline__ void attn_split8(const float (&x)[8], v4u (&p)[3]) {
     }
 }
 
-// acc += A B over 16 k in parts, the small part products first
-__device__ __forceinline__ v16f attn_mfma6(const v4u (&a)[3], const v4u (&b)[3], v16f acc) {
-    const auto f = [](v4u x) { return __builtin_bit_cast(v8bf, x); };
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f(a[2]), f(b[0]), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f(a[0]), f(b[2]), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f(a[1]), f(b[1]), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f(a[1]), f(b[0]), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f(a[0]), f(b[1]), acc, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(f(a[0]), f(b[0]), acc, 0, 0, 0);
+__device__ __forceinline__ v16f attn_mfma(v4u a, v4u b, v16f acc) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), acc, 0, 0, 0);
+}
+// lo + the small part products of A B over 16 k
+__device__ __forceinline__ v16f attn_mfma5(const v4u (&a)[3], const v4u (&b)[3], v16f lo) {
+    lo = attn_mfma(a[2], b[0], lo);
+    lo = attn_mfma(a[0], b[2], lo);
+    lo = attn_mfma(a[1], b[1], lo);
+    lo = attn_mfma(a[1], b[0], lo);
+    return attn_mfma(a[0], b[1], lo);
 }
 
 // 2^40 exp(x) for x <= 8 (0 from about x = -87): 2^t with t = x log2(e) rounded, times exp(x - t ln 2) to first order
@@ -100,7 +104,7 @@ struct AttnLong {
 __device__ __forceinline__ constexpr int attn_key(int r, int h) { return 8 * (r / 4) + 4 * h + r % 4; }
 
 template <int DC, int VT, int NOUT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 3 ? 3 : 2))) void k_attention_long(AttentionArgs a,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 3 ? 3 : DC + VT == 6 ? 1 : 2))) void k_attention_long(AttentionArgs a,
                                                                                                  int vecm, int vecy, int fast,
                                                                                                  int vecq) {
     using T = AttnLong<DC, VT>;
@@ -142,7 +146,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 
     if (threadIdx.x < 2) bad[threadIdx.x] = 0;
 
     float mx = -3.0e38f, top = -__builtin_inff(), sum = 0.f;  // reference, largest score, sum of this lane's half
-    v16f o[VT];
+    v16f o[VT], olo[VT];  // the context: the sums of the large and of the small part products
     auto clear = [&]() {
         mx = -3.0e38f;
         top = -__builtin_inff();
@@ -150,7 +154,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 
 #pragma unroll
         for (int v = 0; v < VT; v++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) o[v][r] = 0.f;
+            for (int r = 0; r < 16; r++) o[v][r] = olo[v][r] = 0.f;
     };
     // the mask elements of this lane's keys of tile kt
     auto load_mask = [&](int kt, float (&mv)[16]) {
@@ -205,7 +209,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 
 #pragma unroll
             for (int v = 0; v < VT; v++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) o[v][r] *= al;
+                for (int r = 0; r < 16; r++) o[v][r] *= al, olo[v][r] *= al;
         }
         float part[4];
 #pragma unroll
@@ -341,6 +345,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 
             load_tile(kn, x0);
             const char *ks = sm[st & 1][kh] + (l & 31) * 16 + h * T::kKStep;
             v16f s;
+            v4u k1[DC];  // the small part products of every chunk, then the large ones
 #pragma unroll
             for (int r = 0; r < 16; r++) s[r] = 0.f;
 #pragma unroll
@@ -349,8 +354,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 
 #pragma unroll
                 for (int q = 0; q < 3; q++)
                     kp[q] = *reinterpret_cast<const v4u *>(ks + q * T::kKPart + 2 * c * T::kKStep);
-                s = attn_mfma6(kp, qp[c], s);
+                k1[c] = kp[0];
+                s = attn_mfma5(kp, qp[c], s);
             }
+#pragma unroll
+            for (int c = 0; c < DC; c++) s = attn_mfma(k1[c], qp[c][0], s);
             scores(kt, s, mv);
             softmax(st == 0, s);
             v4u pp[2][3];
@@ -363,21 +371,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 
             }
             const char *vs = sm[st & 1][kh] + 3 * T::kKPart + (h * 32 + (l & 31)) * 16;
 #pragma unroll
-            for (int v = 0; v < VT; v++)
+            for (int c = 0; c < 2; c++) {  // (the two accumulations of VT tiles side by side: neighbouring MFMAs are independent)
+                v4u vp[VT][3];
 #pragma unroll
-                for (int c = 0; c < 2; c++) {
-                    v4u vp[3];
+                for (int v = 0; v < VT; v++)
 #pragma unroll
                     for (int q = 0; q < 3; q++)
-                        vp[q] = *reinterpret_cast<const v4u *>(vs + q * T::kVPart + (v * 4 + c * 2) * 512);
-                    o[v] = attn_mfma6(vp, pp[c], o[v]);
-                }
+                        vp[v][q] = *reinterpret_cast<const v4u *>(vs + q * T::kVPart + (v * 4 + c * 2) * 512);
+#pragma unroll
+                for (int z = 0; z < 6; z++)
+#pragma unroll
+                    for (int v = 0; v < VT; v++) {
+                        constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+                        v16f &t = z == 5 ? o[v] : olo[v];
+                        t = attn_mfma(vp[v][pa[z]], pp[c][pb[z]], t);
+                    }
+            }
 #pragma unroll
             for (int n = 0; n < T::kItems; n++) store_item(n, x0[n], sm[(st + 1) & 1][kh], &bad[(st + 1) & 1]);
             __syncthreads();
         }
     }
-    float inv = 0.f;
+    float total = 1.f;  // what the context is divided by
     if (again) {
         // on the fp32 MFMA, the tiles in float32: a walk for the maxima and sums, then one with the divided
         // probabilities (at most 1: no sum overflows that the nodes' does not)
@@ -387,7 +402,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 
         for (int n = 0; n < 2 * nt; n++) {
             const bool second = n >= nt;
             const int kt = second ? n - nt : n;
-            if (n == nt) inv = 1.f / (sum + __shfl_xor(sum, 32));
+            if (n == nt) total = sum + __shfl_xor(sum, 32);
             float mv[16];
             load_mask(kt, mv);
             __syncthreads();
@@ -416,15 +431,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 
                 continue;
             }
 #pragma unroll
-            for (int r = 0; r < 16; r++) s[r] = attn_exp40(s[r] - mx) * inv;
+            for (int r = 0; r < 16; r++) s[r] = attn_exp40(s[r] - mx) / total;
 #pragma unroll
             for (int v = 0; v < VT; v++)
 #pragma unroll
                 for (int r = 0; r < 16; r++)
                     o[v] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[attn_key(r, h) * T::kLdV + 32 * v + (l & 31)], s[r], o[v], 0, 0, 0);
         }
-        inv = 1.f;
+        total = 1.f;
     } else {
+#pragma unroll
+        for (int v = 0; v < VT; v++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) o[v][r] = o[v][r] + olo[v][r];
+
         // the second half's context, sum and maxima join the first's (both stages are read: the barrier above)
         float *x = reinterpret_cast<float *>(sm) + (w * 64 + l) * 4;
         constexpr int kRow = 2 * 64 * 4;  // floats of four values of every lane
@@ -454,26 +474,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 
                     o[v][4 * g + 3] = o[v][4 * g + 3] * fa + y.w * fb;
                 }
         }
-        inv = 1.f / (sum + __shfl_xor(sum, 32));
+        total = sum + __shfl_xor(sum, 32);
     }
     if (i >= S || kh) return;
     // a row whose exp(s) are all 0 is 0 / 0 in the reference (its maximum starts at 0)
-    if (top < -103.97208f) inv = __builtin_nanf("");
+    if (top < -103.97208f) total = __builtin_nanf("");
+    // divided with the reciprocal in two floats (the fp32 walk's total is 1 and its context may be infinite)
+    const float inv = 1.f / total, invlo = __builtin_fmaf(-inv, total, 1.f) * inv;
+#pragma unroll
+    for (int v = 0; v < VT; v++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            if (again) o[v][r] *= inv;
+            else o[v][r] = __builtin_fmaf(o[v][r], inv, o[v][r] * invlo);
+        }
     float *Y = a.y + yo + (int64_t)i * a.y_rs;
 #pragma unroll
     for (int v = 0; v < VT; v++)
 #pragma unroll
         for (int g = 0; g < 4; g++) {
             const int dv = 32 * v + 8 * g + 4 * h;
-            float x[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) x[e] = o[v][4 * g + e] * inv;
             if (vecy) {
-                if (dv < DV) *reinterpret_cast<float4 *>(Y + dv) = make_float4(x[0], x[1], x[2], x[3]);
+                if (dv < DV)
+                    *reinterpret_cast<float4 *>(Y + dv) =
+                        make_float4(o[v][4 * g], o[v][4 * g + 1], o[v][4 * g + 2], o[v][4 * g + 3]);
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; e++)
-                    if (dv + e < DV) Y[(int64_t)(dv + e) * a.y_cs] = x[e];
+                    if (dv + e < DV) Y[(int64_t)(dv + e) * a.y_cs] = o[v][4 * g + e];
             }
         }
 }

@@ -104,6 +104,47 @@ def _run(q, k, v, mask, fused=True):
     return g.Output("y").to_numpy()
 
 
+def float32_chain(a, b, ranges=1):
+    """a b with the products added one after another in float32, each exact before it is added, in equal ranges of the
+    inner axis whose sums are added in order."""
+    a64, b64, k = a.astype(np.float64), b.astype(np.float64), a.shape[-1]
+    total = None
+    for r in range(ranges):
+        acc = np.zeros(a.shape[:-1] + (b.shape[-1],), np.float32)
+        for j in range(r * k // ranges, (r + 1) * k // ranges):
+            acc = (acc + a64[..., j:j + 1] * b64[..., j:j + 1, :]).astype(np.float32)
+        total = acc if total is None else total + acc
+    return total
+
+
+@pytest.mark.parametrize("s,d,ranges", [(512, 64, 4), (197, 64, 1), (512, 32, 4), (128, 16, 2)])
+@pytest.mark.parametrize("kind", ["normal", "relu_v", "positive", "sparse_v", "sparse", "few_keys"])
+def test_long_heads_error_is_no_larger_than_the_nodes(hip, s, d, ranges, kind):
+    """Against 64 bits: no further off than float32 products summed in chains (the context's K in the ranges a split
+    product has there), a correctly rounded exponential and a division of every probability."""
+    rng = np.random.default_rng(s + d)
+    q, k, v = (rng.normal(0, 1, (2, s, 4, d)).astype(np.float32) for _ in range(3))
+    mask = np.where(np.arange(s) < s - s // 6, 0.0, -10000.0).astype(np.float32).reshape(1, 1, 1, s)
+    if kind == "relu_v":
+        v = np.maximum(v, 0)
+    elif kind == "positive":
+        q, k, v = (np.maximum(t, 0) for t in (q, k, v))
+    elif kind == "sparse_v":
+        v = v * (rng.random(v.shape) < 0.02)
+    elif kind == "sparse":
+        q, k, v = (t * (rng.random(t.shape) < 0.1) for t in (q, k, v))
+    elif kind == "few_keys":
+        mask = np.where(rng.random((2, 1, 1, s)) < 0.03, 0.0, -10000.0).astype(np.float32)
+        mask[..., 0] = 0
+    q, k, v = (t.astype(np.float32) for t in (q, k, v))
+    qh, kh, vh = (t.transpose(0, 2, 1, 3) for t in (q, k, v))
+    ref, _ = exact(qh, kh, vh, mask, np.float32(8), True)
+    t = float32_chain(qh, kh.transpose(0, 1, 3, 2)) / np.float32(8) + mask
+    e = np.exp((t - np.maximum(t.max(-1, keepdims=True), 0)).astype(np.float64)).astype(np.float32)
+    nodes = float32_chain(e / e.sum(-1, keepdims=True), vh, ranges).transpose(0, 2, 1, 3)
+    assert np.linalg.norm(_run(q, k, v, mask) - ref) <= np.linalg.norm(nodes - ref)
+
+
 @pytest.mark.parametrize("kind", ["plain", "masked_rows", "lowest", "first_keys", "infinite_mask", "tiny_v", "huge_v",
                                   "inf_v", "inf_k", "nan_q", "tiny_qk", "large_scores"])
 def test_long_heads_special_values(hip, kind):
