@@ -22,8 +22,9 @@
 // reciprocal in two floats, after Brisebarre, Muller and Raina 2004; a product for a power of two).  exp(x) is
 // v_exp_f32 of the rounded x log2(e) with the rounding error put back to first order.
 //
-// Values the parts cannot hold (not finite or 2^60 and more in Q, K or V, nonzero below 2^-109 in V, a divisor outside
-// [2^-20, 2^60]) end the walk, and the block runs again on the fp32 MFMA.
+// Values the parts cannot hold (not finite or 2^60 and more in Q, K or V, nonzero below 2^-109 in V) end the walk, and the
+// block runs again on the fp32 MFMA; so do a divisor outside [2^-20, 2^60] and a factor of 2^21 and more, which would
+// bring the parts lost of tiny Q and K back into the scores.
 //
 // Bound: the VALU (16 scores per lane and tile, about 17 instructions each with the splitting, beside 24 or 48 MFMAs
 // of 32 cycles), and at few heads the chain itself.  The three launches it replaces move the scores through memory
@@ -137,8 +138,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 
     const float sv = a.scale ? a.scale[0] : 1.f;
     float sf = sv, sl = 0.f;
     int smode = 0;
+    const uint32_t sb = __builtin_bit_cast(uint32_t, sv), se = (sb >> 23) & 0xffu;
     if (a.scale && a.scale_div) {
-        const uint32_t sb = __builtin_bit_cast(uint32_t, sv), se = (sb >> 23) & 0xffu;
         sf = 1.f / sv;
         sl = __builtin_fmaf(-sf, sv, 1.f) / sv;
         smode = se < 127 - 20 || se > 127 + 60 ? 2 : (sb & 0x7fffffu) ? 1 : 0;
@@ -301,7 +302,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DC + VT <= 
     };
 
     clear();
-    bool again = smode == 2;
+    bool again = smode == 2 || (smode == 0 && se > 127 + 20 && !a.scale_div);
     if (!again) {
         // Q in parts: lane l holds query l % 32, elements 16 c + 8 (l / 32) ..
         v4u qp[DC][3];

@@ -84,19 +84,19 @@ def test_long_heads(hip, case):
     assert [p["op"] for p in g.Profile] == ["Attention"]
 
 
-def _run(q, k, v, mask, fused=True):
-    """Projection-layout inputs [b, s, h, d] through the transposed views, the mask an input, scale 8."""
+def _run(q, k, v, mask, fused=True, scale=("Div", 8.0)):
+    """Projection-layout inputs [b, s, h, d] through the transposed views, the mask an input, scores divided by 8."""
     b, s, h, d = q.shape
     nodes = [W.node("Transpose", ["q"], ["qt"], "tq", perm=[0, 2, 1, 3]),
              W.node("Transpose", ["k"], ["kt"], "tk", perm=[0, 2, 3, 1]),
              W.node("Transpose", ["v"], ["vt"], "tv", perm=[0, 2, 1, 3]),
-             W.node("MatMul", ["qt", "kt"], ["sc"], "scores"), W.node("Div", ["sc", "c"], ["sd"], "scale"),
+             W.node("MatMul", ["qt", "kt"], ["sc"], "scores"), W.node(scale[0], ["sc", "c"], ["sd"], "scale"),
              W.node("Add", ["sd", "mask"], ["t"], "add"), W.node("Softmax", ["t"], ["p"], "softmax", axis=-1),
              W.node("MatMul", ["p", "vt"], ["ctx"], "context"),
              W.node("Transpose", ["ctx"], ["y"], "ty", perm=[0, 2, 1, 3])]
     ins = {"q": q, "k": k, "v": v, "mask": mask}
     g = Model.Load(W.model(nodes, [(n, np.float32, a.shape) for n, a in ins.items()], [("y", np.float32, ())],
-                           [("c", np.array(8.0, np.float32))]))
+                           [("c", np.array(scale[1], np.float32))]))
     if fused:
         g.Fuse()
         assert [n.Op for n in g.Nodes] == ["Attention"]
@@ -203,3 +203,18 @@ def test_long_heads_random(hip):
         ref, bar = exact(*(t.transpose(0, 2, 1, 3) for t in (q, k, v)), mask, np.float32(8), True)
         got = _run(q, k, v, mask)
         assert np.all(np.abs(got - ref) <= bar), (b, h, s, d, float((np.abs(got - ref) / bar).max()))
+
+
+@pytest.mark.parametrize("scale", [("Mul", 1e37), ("Mul", -3e20), ("Mul", 1e6), ("Div", 1e-30), ("Div", -7.3), ("Mul", 1e-20)])
+def test_long_heads_scales(hip, scale):
+    """Scale constants far from 1 over operands that bring the scores back to a few units, tiny ones included: the
+    unfused graph's values within 1e-5 of the context's magnitude."""
+    rng = np.random.default_rng(41)
+    b, s, h, d = 1, 100, 3, 64
+    q, k, v = (rng.normal(0, 1, (b, s, h, d)).astype(np.float32) for _ in range(3))
+    f = 0.125 / abs(scale[1] if scale[0] == "Mul" else 1 / scale[1])
+    q = (q * (f if f < 1 else f ** 0.5)).astype(np.float32)
+    k = (k * (1 if f < 1 else f ** 0.5)).astype(np.float32)
+    mask = np.where(np.arange(s) < 90, 0.0, -10000.0).astype(np.float32).reshape(1, 1, 1, s)
+    got, ref = _run(q, k, v, mask, scale=scale), _run(q, k, v, mask, fused=False, scale=scale)
+    assert np.all(np.abs(got - ref) <= 1e-5 * np.abs(v).max())
