@@ -527,10 +527,33 @@ static void attention_long_launch(const AttentionArgs &a, int vecm, int vecy, hi
     }
 }
 
+// Whether heads run here: kernel sizes, and the estimated time (us) below that of the three launches.  Here: rounds of
+// blocks of 64 rows, `per` of them on a CU; a block takes `block` and, per step of 64 keys, `step` (`inexact` times that
+// where D or DV is not the tile's and the loads are the general ones), `more` for every other block on its CU.  Each step
+// is a chain of products, maximum, exponentials and products, so few heads over many keys wait for it where the three
+// launches spread over the chip (128 rows and 1024 keys of one head of 64: 56.5 against 21.7 us).  The three launches: `nodes`, then by the scores' elements, their rows 16-byte aligned or
+// not (four passes over them), and, where the context's K does not split, by the keys.  Fitted to 577 shapes (heads of 16
+// to 64, 1 to 384 of them, 65 to 2048 rows and 73 to 2048 keys): what it picks is within 10% of the faster one in 574.
 bool attention_long_fits(const AttentionArgs &a) {
-    const int64_t waves = a.batch * ((a.s + 31) / 32);
-    return a.s > 64 && a.sk > kAttentionLongKeys && a.d >= 1 && a.d <= 64 && a.dv >= 1 && a.dv <= 64 &&
-           a.batch >= 1 && a.batch * ((a.s + 63) / 64) <= 0x7fffffff && (waves >= 128 || a.sk <= 1024);
+    if (a.s <= 64 || a.sk <= kAttentionLongKeys || a.d < 1 || a.d > 64 || a.dv < 1 || a.dv > 64 || a.batch < 1) return false;
+    const int64_t blocks = a.batch * ((a.s + 63) / 64);
+    if (blocks > 0x7fffffff) return false;
+    struct Cost {
+        double launch, block, step, more, inexact, tail;
+        int per;
+    };
+    static const Cost kCost[3] = {{8.7, 4.1, 1.6, 1.2, 1.5, 0.4, 3}, {5.8, 8.7, 1.6, 1.6, 1.5, 0.6, 2}, {5.2, 9.6, 2.6, 0, 1.7, 1.2, 1}};
+    const bool wide = a.d > 32, tall = a.dv > 32;
+    const Cost &c = kCost[wide + tall];
+    const double steps = (double)((a.sk + 63) / 64), fixed = c.block + (a.sk % 32 ? c.tail : 0);
+    const double step = c.step * (a.d == (wide ? 64 : 32) && a.dv == (tall ? 64 : 32) ? 1 : c.inexact);
+    const int64_t per_cu = (blocks + 255) / 256, rest = per_cu % c.per;
+    double here = c.launch + (double)(per_cu / c.per) * (fixed + steps * (step + c.more * (c.per - 1)));
+    if (rest) here += fixed + steps * (step + c.more * (double)(rest - 1));
+    const double scores = 1e-6 * (double)a.batch * a.s * a.sk;
+    const double nodes = wide || tall ? 19 + scores * (a.sk % 4 ? 13.9 : 4.5) + (a.sk % 64 ? 0.023 * a.sk : 0) + (a.sk % 4 ? 4.4 : 0)
+                                      : 18.5 + scores * (a.sk % 4 ? 11.5 : 3.8) + (a.sk % 64 ? 0.032 * a.sk : 0);
+    return here < nodes;
 }
 
 hipError_t launch_attention_long(const AttentionArgs &a, hipStream_t s) {

@@ -80,7 +80,8 @@ int api_matmul_permuted(const lx_tensor *A, const int *a_perm, const lx_tensor *
 // probabilities x transpose(V, v_perm) stored as transpose(context, y_perm) into Y, in one launch.  Float, equal
 // batch axes.  Rows, keys and head widths of at most kAttentionMax: bit for bit the MatMulPermuted,
 // ScaleAddSoftmax (AddSoftmax without a scale) and MatMulPermuted nodes it replaces.  Longer heads of widths of
-// at most 64 (attention_long_fits): their result with the sums in another order.  LX_ERR_NOT_SUPPORTED (no
+// at most 64, where one launch is estimated the faster form (attention_long_fits): their result with the sums in another
+// order.  LX_ERR_NOT_SUPPORTED (no
 // message) otherwise.
 int api_attention(const lx_tensor *Q, const int *q_perm, const lx_tensor *K, const int *k_perm,
                   const lx_tensor *scale, int scale_div, const lx_tensor *mask, int32_t axis, const lx_tensor *V,

@@ -169,10 +169,10 @@ struct AttentionArgs {
     int32_t scale_div;
 };
 hipError_t launch_attention(const AttentionArgs &a, hipStream_t s);
-// Longer heads, of more than 64 rows and more than kAttentionLongKeys keys and widths of at most 64, in one launch: the
+// Longer heads, of more than 64 rows and more than kAttentionLongKeys keys and widths of at most 64, in one launch where
+// that is estimated the faster form (attention_long_fits: enough heads for the chip, or few keys): the
 // same result with the sums of the products and of the Softmax in another order (the scores are never in memory).
-// Up to kAttentionLongKeys keys the three launches stay: a head of 65 keys pads to three tiles of 32.  A few heads
-// over more than 1024 keys (fewer than 128 waves of 32 rows) stay with them too: each wave walks every key.
+// Up to kAttentionLongKeys keys the three launches stay: a head of 65 keys pads to three tiles of 32.
 constexpr int kAttentionLongKeys = 72;
 bool attention_long_fits(const AttentionArgs &a);
 hipError_t launch_attention_long(const AttentionArgs &a, hipStream_t s);
