@@ -33,12 +33,14 @@ def check(a, b, got=None):
     assert np.all(err <= bar * mag + 2.0 ** -140), float((err / (mag + 1e-300)).max())
 
 
-# every tile (128x128; 128x64; 64x64 several per CU; 64x64 with loading waves), each with whole step pairs, a K tail in
-# 16-byte loads (K % 4 == 0), scalar loads (odd K) and edges in both directions; K ranges of a split product; a batch
-SHAPES = [(256, 256, 128), (4096, 256, 1024), (4096, 384, 384), (1000, 320, 4100), (788, 768, 768), (129, 256, 65),
-          (2000, 260, 2020), (700, 333, 260), (127, 257, 33), (2048, 1001, 1030), (1, 2048, 4096), (300, 1000, 36),
-          (512, 768, 768), (64, 4096, 64), (5, 300, 7),
-          (1024, 512, 512), (1100, 516, 512), (100, 600, 70), (1100, 384, 960)]  # a CU per tile: from K = 512
+# Every form of the kernel: the tiles with whole pairs of steps (128x128, 128x64, 64x64 several per CU, 64x64 with loading
+# waves), K tails in 16-byte loads (128x128 and 64x64) and in scalar ones (both), the ranges of a split product
+FORMS = [(4096, 256, 1024), (1100, 384, 960), (4096, 256, 1152), (1024, 512, 512), (1536, 516, 1600), (600, 516, 516),
+         (1500, 533, 1601), (256, 533, 70), (640, 3072, 640)]
+# and edges in both directions, single rows and few columns, the first K with a CU per tile
+SHAPES = FORMS + [(4096, 384, 384), (1000, 320, 4100), (788, 768, 768), (129, 516, 65), (2000, 260, 2020), (700, 533, 260),
+                  (127, 513, 33), (2048, 1001, 1030), (1, 4100, 500), (300, 1000, 36), (700, 768, 768), (5, 700, 37),
+                  (1100, 516, 512), (100, 600, 70)]
 
 
 @pytest.mark.parametrize("m,k,n", SHAPES)
@@ -50,21 +52,27 @@ def test_parts_tiles_and_edges(hip, m, k, n):
 
 def test_parts_batches(hip):
     rng = np.random.default_rng(3)
-    for sa, sb in [((3, 1, 130, 256), (1, 2, 256, 132)), ((70, 65, 300), (70, 300, 67))]:
+    for sa, sb in [((30, 1, 130, 256), (1, 2, 256, 132)), ((70, 65, 300), (70, 300, 67))]:
         check(rng.standard_normal(sa).astype(np.float32), rng.standard_normal(sb).astype(np.float32))
 
 
-@pytest.mark.parametrize("m,k,n", [(260, 512, 516), (256, 533, 70), (1090, 333, 1000)])
-@pytest.mark.parametrize("kind", ["tiny", "tiny_times_huge", "huge", "mixed", "not_finite"])
+@pytest.mark.parametrize("m,k,n", FORMS + [(1090, 333, 1000)])
+@pytest.mark.parametrize("kind", ["tiny", "tiny_times_huge", "one_tiny", "huge", "mixed", "not_finite"])
 def test_parts_of_extreme_values(hip, m, k, n, kind):
-    """Values whose parts bf16 cannot hold take the fp32 MFMA: subnormal operands, subnormal times huge, values that
-    round to an infinite bf16, rows over 45 decades, and infinities and NaN (the same pattern as float32's)."""
+    """Values whose parts bf16 cannot hold take the fp32 MFMA: subnormal operands, subnormal times huge, a row's only
+    product that of a subnormal beside larger values, values that round to an infinite bf16, rows over 45 decades, and
+    infinities and NaN (the same pattern as float32's)."""
     rng = np.random.default_rng(7)
     a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
     if kind == "tiny":
         a = (a * 1e-36).astype(np.float32)
     elif kind == "tiny_times_huge":
         a, b = (a * 1e-41).astype(np.float32), (b * np.float32(1e20)).astype(np.float32)
+    elif kind == "one_tiny":
+        a[::5], a[::5, 7], a[::5, 9] = 0, 1e-41, 1
+        b[7], b[9] = b[7] * np.float32(1e15), 0
+        b[:, ::7], b[7, ::7], b[9, ::7] = 0, 1e-41, 1  # columns likewise
+        a[1::5, 7], a[1::5, 9] = 1e15, 0
     elif kind == "huge":
         a[::3, 5] = np.float32(3.4e38)
         b[5, :] = 0.25
@@ -97,7 +105,7 @@ def float32_chain(a, b):
 
 
 # 128x64, 64x64, 128x128 tiles, loading waves, a split product, scalar loads with a tail
-@pytest.mark.parametrize("m,k,n", [(1100, 384, 960), (600, 516, 516), (788, 768, 2500), (700, 768, 768), (8, 4096, 4096),
+@pytest.mark.parametrize("m,k,n", [(1100, 384, 960), (600, 516, 516), (788, 768, 2500), (700, 768, 768), (640, 3072, 640),
                                    (1090, 333, 1000)])
 @pytest.mark.parametrize("dense", [1.0, 0.5, 0.1, 0.02, "both", "positive", "small"])
 def test_parts_error_is_no_larger_than_a_float32_chain(hip, m, k, n, dense):
@@ -179,7 +187,22 @@ def test_parts_results_do_not_depend_on_the_tile(hip):
         assert np.array_equal(part.view(np.uint32), whole[rows, cols].view(np.uint32))
 
 
-@pytest.mark.parametrize("s,d", [(512, 256), (512, 320), (301, 515)])
+def test_parts_of_a_long_k_do_not_depend_on_the_tile(hip):
+    """K = 512: 64x64 tiles whole, its parts 128x128, 128x64 and 64x64 with loading waves; rows of subnormals and a few
+    values that are not finite run on the fp32 MFMA in each."""
+    rng = np.random.default_rng(12)
+    a, b = rng.standard_normal((4096, 512)).astype(np.float32), rng.standard_normal((512, 1152)).astype(np.float32)
+    a[10] *= np.float32(1e-38)
+    a[900, 500], a[70, 3], b[4, 500], b[300, 20] = np.nan, np.inf, np.float32(1e-40), -np.inf
+    whole = mm(a, b)
+    for rows, cols in [(slice(0, 2048), slice(0, 1152)), (slice(0, 1024), slice(0, 1152)), (slice(0, 1024), slice(0, 512))]:
+        part = mm(np.ascontiguousarray(a[rows]), np.ascontiguousarray(b[:, cols]))
+        nan = np.isnan(whole[rows, cols])
+        assert np.array_equal(np.isnan(part), nan)
+        assert np.array_equal(part[~nan].view(np.uint32), whole[rows, cols][~nan].view(np.uint32))
+
+
+@pytest.mark.parametrize("s,d", [(640, 256), (512, 320), (301, 515)])
 def test_parts_of_a_right_operand_by_columns(hip, s, d):
     """A transposed right operand folded into the product is read by columns: bit for bit the Transpose and MatMul
     nodes (128x128 and 64x64 tiles, 16-byte and scalar loads, a K tail)."""
