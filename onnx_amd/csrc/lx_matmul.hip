@@ -1051,19 +1051,23 @@ static bool f32_b3(const MatMulArgs &p, int kr) {
 // The block tile: the least estimated time.  A block takes `fixed` us (first stage, check, stores) and per step of 16 k
 // `lone` us when it has a CU to itself, `full` us per block in a launch of several blocks per CU (r of them at once, else
 // one after another): rounds of r blocks, then the rest.  Fitted to [4096, 384..3072] x [.., 384..3072], [788, ..],
-// 1024^3 to 2048^3 and 12 batches of 384^3 and 512^3, where the tile it picks is the fastest of the four or within 4%.
+// 1024^3 to 2048^3 and 12 batches of 384^3 and 512^3, where the tile it picks is the fastest or within 4%.  128x128 has
+// two forms: eight waves of 64x32, one block per CU, and four of 64x64, two of them (255 registers), whose first stage and
+// epilogue the other block covers: [4096,768]x[768,3072] 118 against 111 us, [4096,3072]x[3072,768] (192 tiles, a block
+// per CU) 118 against 130.
 static int b3_tile(const MatMulArgs &p, bool only_general) {
     struct B3Tile {
         int bm, bn, r;
         double fixed, lone, full;
     };
     static const B3Tile cand[] = {{128, 128, 1, 2.9, 0.58, 0.62}, {128, 64, 1, 1.8, 0.35, 0.44},
-                                  {64, 64, 3, 1.5, 0.27, 0.25}, {64, 64, 1, 1.0, 0.21, 0.28}};
+                                  {64, 64, 3, 1.5, 0.27, 0.25}, {64, 64, 1, 1.0, 0.21, 0.28},
+                                  {128, 128, 2, 2.5, 0.62, 0.64}};
     const double steps = (double)((p.k + 15) / 16);
     int best = 0;
     double cost = 0;
-    for (int i = 0; i < 4; i++) {
-        if (only_general && (i == 1 || i == 3)) continue;
+    for (int i = 0; i < 5; i++) {
+        if (only_general && i != 0 && i != 2) continue;
         const B3Tile &c = cand[i];
         const int64_t tiles = (int64_t)((p.m + c.bm - 1) / c.bm) * ((p.n + c.bn - 1) / c.bn) * p.batch;
         const int64_t per_cu = (tiles + 255) / 256, rounds = per_cu / c.r, rest = per_cu - rounds * c.r;
@@ -1116,6 +1120,7 @@ static void launch_f32_b3(const float *a, const float *b, float *c, const MatMul
     }
     switch (tile) {
     case 0: b3_launch<128, 128, 2, 4, 0, 1, 2, true, false, false>(a, b, c, p, vec, s); break;
+    case 4: b3_launch<128, 128, 2, 2, 0, 1, 2, true, false, false>(a, b, c, p, vec, s); break;
     case 1: b3_launch<128, 64, 4, 2, 0, 2, 2, true, false, false>(a, b, c, p, vec, s); break;
     case 2: b3_launch<64, 64, 2, 2, 0, 2, 3, true, false, false>(a, b, c, p, vec, s); break;
     default: b3_launch<64, 64, 2, 2, 8, 2, 3, true, false, false>(a, b, c, p, vec, s); break;
