@@ -28,8 +28,8 @@
 //
 // Bound: the VALU (16 scores per lane and tile, about 17 instructions each with the splitting, beside 24 or 48 MFMAs
 // of 32 cycles), and at few heads the chain itself.  The three launches it replaces move the scores through memory
-// four times: [8,12,512,512] heads of 32 took 34 + 32 + 25 us against 38 here, [4,12,197,197] heads of 64
-// 24 + 8.5 + 18 against 24.
+// four times: [8,12,512,512] heads of 32 took 34 + 32 + 25 us against 42 here, [4,12,197,197] heads of 64
+// 24 + 8.5 + 18 against 26.6 (94 and 54 us a captured graph, 45 and 27).
 #include <hip/hip_runtime.h>
 
 #include "lx_device.h"
@@ -531,8 +531,8 @@ static void attention_long_launch(const AttentionArgs &a, int vecm, int vecy, hi
 // blocks of 64 rows, `per` of them on a CU; a block takes `block` and, per step of 64 keys, `step` (`inexact` times that
 // where D or DV is not the tile's and the loads are the general ones), `more` for every other block on its CU.  Each step
 // is a chain of products, maximum, exponentials and products, so few heads over many keys wait for it where the three
-// launches spread over the chip (128 rows and 1024 keys of one head of 64: 56.5 against 21.7 us).  The three launches: `nodes`, then by the scores' elements, their rows 16-byte aligned or
-// not (four passes over them), and, where the context's K does not split, by the keys.  Fitted to 577 shapes (heads of 16
+// launches spread over the chip (128 rows and 1024 keys of one head of 64: 56.5 against 21.7 us).  The three launches:
+// `nodes`, then by the scores' elements, their rows 16-byte aligned or not (four passes over them), and, where the context's K does not split, by the keys.  Fitted to 577 shapes (heads of 16
 // to 64, 1 to 384 of them, 65 to 2048 rows and 73 to 2048 keys): what it picks is within 10% of the faster one in 574.
 bool attention_long_fits(const AttentionArgs &a) {
     if (a.s <= 64 || a.sk <= kAttentionLongKeys || a.d < 1 || a.d > 64 || a.dv < 1 || a.dv > 64 || a.batch < 1) return false;

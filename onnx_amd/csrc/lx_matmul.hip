@@ -1,15 +1,19 @@
 // lx_matmul.hip -- MatMul on gfx950 (Tensor<T>.MatMul, TensorOps.cs:504-806,
 // via CPUExecutionProvider.MatMul, CPUExecutionProvider.cs:359-378).
 //
-// float : K ranges of 256 and more (N above 32): every operand in three bf16
-//         parts on v_mfma_f32_32x32x16_bf16 (k_matmul_f32_b3), closer to 64
-//         bits than float32 products and 2.2 times the rate.  Shorter ones:
+// float : K ranges of 512 and more, and of 256 and more over more than 256
+//         tiles of 64x64, with N above 32 (f32_b3): every operand in three
+//         bf16 parts on v_mfma_f32_32x32x16_bf16 (k_matmul_f32_b3), closer to
+//         64 bits than float32 products and 2.2 times the rate.  The others,
+//         and ranges of up to 1024 of a split product:
 //         v_mfma_f32_32x32x2f32 (fp32 products, fp32 accumulation), summed in
 //         one order by two kernels: K a multiple of 64 with aligned operands
 //         through a ring of LDS stages filled by direct-to-LDS loads
 //         (k_matmul_f32_dl), otherwise double-buffered LDS fed from registers
 //         one K step ahead (k_matmul_f32).  Block tiles from 64x64 to 128x128
-//         chosen per shape, K step 16, four waves.
+//         chosen per shape, K step 16, four waves.  Split products of at most
+//         64 rows in ranges of 64: one launch on the VALU in that order
+//         (k_matmul_small).
 // double: v_mfma_f64_16x16x4f64, 64x64 block tile, four waves of 32x32.
 // int32 : exact two's-complement products as ten int8 digit products on
 //         v_mfma_i32_32x32x32_i8 (small products of K up to 96: on the VALU).
@@ -642,7 +646,8 @@ static void launch_f32_dl(const float *a, const float *b, float *c, const MatMul
 // of the splitting (15 VALU instructions per pair of elements) and of LDS, so each element is split once per block,
 // on its way from global memory to LDS, and the splitting, the LDS accesses and the loads are dealt out between the
 // MFMAs one by one (in runs they stalled the wave's MFMAs: [4096,3072]x[3072,768] 208 us with the phases one after
-// another, 130 with fragments a step ahead, 112 dealt out evenly with eight waves).  Stage layout: per 16-k sub-step
+// another, 130 with fragments a step ahead, 112 dealt out evenly with eight waves; 118 since the small products have their
+// own accumulator).  Stage layout: per 16-k sub-step
 // and part, [k half][row] chunks of eight bf16, the halves 64 bytes apart modulo 256: the 16-byte fragment reads and
 // the writes are free of bank conflicts.  Two stages: step t multiplies the fragments read during step t - 1, reads
 // those of step t + 1, writes the parts of step t + 2 into the stage they left and loads step t + 4.
@@ -685,8 +690,8 @@ __device__ __noinline__ v16f f32_tile(const float *A, const float *B, int M, int
 // BM x BN tile, WM x WN multiplying waves, KS sub-steps of 16 per step, WE waves per SIMD.  PW: loading waves that
 // load and split for them (0: every wave does both).  A block alone on its CU is bound by its waves' issue slots, not
 // by the matrix unit: eight loading waves beside the four of a 64x64 tile take [788,3072]x[3072,768] (156 tiles) from
-// 57 to 44 us; with several blocks per CU, or 128x128 tiles, both forms run alike or the joint one faster ([4096,768]x
-// [768,3072] 107 against 120 us).  VEC: 16-byte loads along K (the rows
+// 58 to 45 us; with 128x128 tiles both forms run alike ([4096,3072]x[3072,768] 118 in eight joint waves, 118 to 126 with
+// eight or four loading ones).  VEC: 16-byte loads along K (the rows
 // of A, and of B by columns, 16-byte aligned).  TAIL: the K range is no whole number of step pairs (past it the loads
 // clamp to the last step's and their elements are zeroed).  vc: 16-byte epilogue.  SPLIT as in k_matmul_f32_dl.
 template <int BM, int BN, int WM, int WN, int PW, int KS, int WE, bool VEC, bool TAIL, bool BT, bool GELU,
@@ -1036,8 +1041,10 @@ constexpr int kB3MinK = 256, kB3LoneK = 512, kB3SplitK = 1024;
 // Whether a K range of kr goes to k_matmul_f32_b3: kB3MinK or more, N above 32 (a context product of 32-wide heads is
 // bound by its loads: [96,512,512]x[96,512,32] 24 us on the fp32 MFMA, 26 in parts), and strides whose offsets within
 // a tile and a step stay below 2^31 bytes (rows of up to 8 MB; longer ones keep the fp32 MFMA).  A range below kB3LoneK
-// whose 64x64 tiles (f32_tiles) find a CU each keeps the fp32 MFMA too: the parts' first stage and last check cost 1.2 us more than a block of so few steps gains
-// (six batches of 384^3 11.8 against 10.2 us; [1024,512]x[512,512], the first on the other side, 11.0 in both).  The
+// whose 64x64 tiles (f32_tiles, whichever tile b3_tile then takes) find a CU each keeps the fp32 MFMA too: the parts' first
+// stage and last check cost 1.2 us more than a block of so few steps gains
+// (six batches of 384^3 11.8 against 10.2 us; past the line [4096,384]x[384,384] 14.9 against 15.9, 12 batches of 384^3
+// 17.4 / 17.0, [1024,512]x[512,512] 11.0 in both).  The
 // ranges of a split product, at most one block per CU and mostly of few rows, keep it up to kB3SplitK: there the parts'
 // 4-byte loads of B count too (ranges of 512: [60,2560]x[2560,4096] 18.0 us in parts, 16.5; 768: [256,3072]x[3072,768]
 // 18.9, 18.3; 1024: [384,3072]x[3072,768] 22.6, 22.5; 1536: [640,3072]x[3072,640] 29.3, 30.1).
@@ -1147,8 +1154,8 @@ static void launch_f32_parts(const float *a, const float *b, float *c, const Mat
 // from LDS, each range padded by four floats (the four ranges of a wave read different banks).  The partials then meet
 // in LDS and are summed in range order with the epilogue, exactly as k_matmul_split_sum does.
 // Bound: launches and memory latency.  5.1 us a product ([8,1536]x[1536,384] and the like) in place of 4.3 for the
-// tiles and 3.7 to 5.4 for the sum; a captured encoder of 12 layers of 384 at 8 tokens 510 -> 400 us, at 32 530 -> 430,
-// at 64 584 -> 512.
+// tiles and 3.7 to 5.4 for the sum; a captured encoder of 12 layers of 384, replayed in a row, at 8 tokens 513 -> 400 us,
+// at 32 540 -> 442, at 64 585 -> 512.
 constexpr int kSmallR = 4, kSmallC = 16, kSmallRanges = 64;
 
 template <bool GELU>
@@ -1412,7 +1419,7 @@ static void launch_f64(const double *a, const double *b, double *c, const MatMul
 // Modulo 2^32 an int32 is four signed base-256 digits, x = d0 + 2^8 d1 + 2^16 d2 + 2^24 d3, -128 <= d <= 127: the
 // bytes of (x + 0x80808080) ^ 0x80808080.  A product is then the ten digit products of weight below 2^32, those of one
 // weight summed in one int32 accumulator by v_mfma_i32_32x32x32_i8: exact below 2^31, i.e. for 2^15 k (up to four
-// products of 2^14 each per k), so every kFoldK the four accumulators are folded into the wrapping result.
+// products of 2^14 each per k), so every kI32Fold the four accumulators are folded into the wrapping result.
 //
 // k_matmul_i32: 64x64 tile, four waves of 32x32 (four accumulators each), K steps of 64.  Elements go from global memory
 // to registers one step ahead, are split (two instructions, then a 4x4 byte transpose) and written to LDS as four digit
@@ -1796,7 +1803,7 @@ hipError_t launch_matmul(int dtype, const void *a, const void *b, void *c, const
             launch_f32_b3(fa, fb, fc, p, vec, s);
             return hipGetLastError();
         }
-        // K below kB3MinK.  Block tile: among the tiles that give each of the 256 CUs two or more blocks (a lone block
+        // What f32_b3 leaves.  Block tile: among the tiles that give each of the 256 CUs two or more blocks (a lone block
         // per CU leaves its barrier and load latencies unhidden: measured 93 against 104 TF/s for
         // [4096,3072]x[3072,768]), the one whose busiest CU has the least work -- ceil(blocks / 256)
         // blocks, each costing its area over the tile's relative efficiency; 64x64 when none does
