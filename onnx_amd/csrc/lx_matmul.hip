@@ -974,9 +974,10 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
         const bool la = amin[wr + 32 * i + (l & 31)] < kLossy;
 #pragma unroll
         for (int j = 0; j < NT; j++) {
-            // whether the tile can hold such a result: one is not finite or nonzero below 2^-120, a row or column
-            // holds a value below 2^-109, or the largest of a row and of a column multiply to less than 2^-120 (lane l:
-            // row and column l % 32)
+            // whether the tile can hold such a result: one is not finite or nonzero below 2^-120; or (bounds over the
+            // tile's rows and columns; lane l holds row and column l % 32) small beside a column where a row holds a
+            // value below 2^-109, or the other way round; or zero with no product of 2^-120.  Element by element only
+            // then: probabilities of a Softmax have such rows all over.
             float top = 0.f;
             uint32_t low = ~0u;
 #pragma unroll
@@ -987,13 +988,24 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) __attribute__((amdgpu_waves_pe
                 top = __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(v0), fabsf(v1)), top);
                 low = min(min((__builtin_bit_cast(uint32_t, v0) << 1) - 1u, (__builtin_bit_cast(uint32_t, v1) << 1) - 1u), low);
             }
-            const uint32_t lc = bmin[wc + 32 * j + (l & 31)];
+            const bool lc = bmin[wc + 32 * j + (l & 31)] < kLossy;
             const float c0 = __builtin_bit_cast(float, bmax[wc + 32 * j + (l & 31)]);
-            if (!__any(!(top < __builtin_inff()) || low < kUnder || la || lc < kLossy)) {
-                if (!__any((ra != 0.f && ra < 0x1p-60f) || (c0 != 0.f && c0 < 0x1p-60f))) continue;
-                float rm = ra != 0.f ? ra : __builtin_inff(), cm = c0 != 0.f ? c0 : __builtin_inff();
-                for (int o = 1; o < 32; o *= 2) rm = fminf(rm, __shfl_xor(rm, o)), cm = fminf(cm, __shfl_xor(cm, o));
-                if (!__any(rm * cm < 0x1p-120f)) continue;
+            if (!__any(!(top < __builtin_inff()) || low < kUnder)) {
+                const bool lossy_row = __any(la), lossy_col = __any(lc);
+                if (!lossy_row && !lossy_col && !__any((ra != 0.f && ra < 0x1p-60f) || (c0 != 0.f && c0 < 0x1p-60f))) continue;
+                const auto larger = [](float x, float y) { return fmaxf(x, y); };
+                const auto smaller = [](float x, float y) { return fminf(x, y); };
+                const float rx = wave_reduce_dpp(ra, larger), cx = wave_reduce_dpp(c0, larger);
+                const float rn = wave_reduce_dpp(ra != 0.f ? ra : __builtin_inff(), smaller);
+                const float cn = wave_reduce_dpp(c0 != 0.f ? c0 : __builtin_inff(), smaller);
+                const float lim = fmaxf(lossy_row ? cx : 0.f, lossy_col ? rx : 0.f) * 0x1p-96f;
+                bool zero = false;
+#pragma unroll
+                for (int r = 0; r < 16; r++) zero = zero || acc[i][j][r] == 0.f;
+                const bool none = low == ~0u;  // all of this lane's are zero
+                if (!__any((!none && __builtin_bit_cast(float, (low + 1u) >> 1) < lim) ||
+                           (zero && (lim > 0.f || rn * cn < 0x1p-120f))))
+                    continue;
             }
             uint32_t again = 0;
 #pragma unroll
