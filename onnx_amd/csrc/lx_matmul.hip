@@ -1,8 +1,8 @@
 // lx_matmul.hip -- MatMul on gfx950 (Tensor<T>.MatMul, TensorOps.cs:504-806,
 // via CPUExecutionProvider.MatMul, CPUExecutionProvider.cs:359-378).
 //
-// float : K ranges of 512 and more, and of 256 and more over more than 256
-//         tiles of 64x64, with N above 32 (f32_b3): every operand in three
+// float : K ranges above 512, and of 256 and more over more than 256
+//         tiles of 64x64, with N above 32 (but see f32_b3): every operand in three
 //         bf16 parts on v_mfma_f32_32x32x16_bf16 (k_matmul_f32_b3), closer to
 //         64 bits than float32 products and 2.2 times the rate.  The others,
 //         and ranges of up to 1024 of a split product:
@@ -1049,14 +1049,18 @@ static int64_t f32_tiles(const MatMulArgs &p, bool fold) {
     return fold ? (p.m * batch + 63) / 64 * cols : ((int64_t)p.m + 63) / 64 * cols * batch;
 }
 
-constexpr int kB3MinK = 256, kB3LoneK = 512, kB3SplitK = 1024;
+constexpr int kB3MinK = 256, kB3LoneK = 512, kB3SplitK = 1024, kB3NarrowK = 1024;
 // Whether a K range of kr goes to k_matmul_f32_b3: kB3MinK or more, N above 32 (a context product of 32-wide heads is
 // bound by its loads: [96,512,512]x[96,512,32] 24 us on the fp32 MFMA, 26 in parts), and strides whose offsets within
-// a tile and a step stay below 2^31 bytes (rows of up to 8 MB; longer ones keep the fp32 MFMA).  A range below kB3LoneK
+// a tile and a step stay below 2^31 bytes (rows of up to 8 MB; longer ones keep the fp32 MFMA).  A range of up to kB3LoneK
 // whose 64x64 tiles (f32_tiles, whichever tile b3_tile then takes) find a CU each keeps the fp32 MFMA too: the parts' first
-// stage and last check cost 1.2 us more than a block of so few steps gains
-// (six batches of 384^3 11.8 against 10.2 us; past the line [4096,384]x[384,384] 14.9 against 15.9, 12 batches of 384^3
-// 17.4 / 17.0, [1024,512]x[512,512] 11.0 in both).  The
+// stage and last check cost 1.2 us more than a block of so few steps gains (six batches of 384^3 11.8 against 10.2 us, 12
+// of [512,512]x[512,128] 12.3 / 11.9; past the line [4096,384]x[384,384] 14.9 / 15.9, 12 batches of 384^3 17.4 / 17.0,
+// [788,768]x[768,768] 14.7 / 15.1).  So does a K below kB3NarrowK over 64 columns (the context of 64-wide heads: a left
+// operand that is read once) unless a CU has two tiles: [96,512,512]x[96,512,64] 35.3 / 32.4, [48,197,512]x[48,512,64]
+// 12.7 / 12.0; [192,128,512]x[192,512,64] 18.2 / 20.7, [96,512,1024]x[96,1024,64] 61.5 / 61.3.  Where the direct-load fp32
+// kernel does not take the operands (K no multiple of 64, N no multiple of 4 or below 64) the other one is slower, and K
+// of 512 and N of 33 to 64 run in parts: [12,512,512]x[12,512,65] 14.1 / 33.9, [48,197,512]x[48,512,40] 12.0 / 18.2.  The
 // ranges of a split product, at most one block per CU and mostly of few rows, keep it up to kB3SplitK: there the parts'
 // 4-byte loads of B count too (ranges of 512: [60,2560]x[2560,4096] 18.0 us in parts, 16.5; 768: [256,3072]x[3072,768]
 // 18.9, 18.3; 1024: [384,3072]x[3072,768] 22.6, 22.5; 1536: [640,3072]x[3072,640] 29.3, 30.1).
@@ -1064,7 +1068,10 @@ static bool f32_b3(const MatMulArgs &p, int kr) {
     const int64_t lim = kMatMulPartsRow;
     if (kr < kB3MinK || p.n <= 32 || p.lda > lim || p.ldb > lim || p.k > (1 << 24)) return false;
     if (kr < p.k) return kr > kB3SplitK;
-    return kr >= kB3LoneK || f32_tiles(p, true) > 256;
+    const int64_t tiles = f32_tiles(p, true);
+    const bool direct = kr % 64 == 0 && p.n % 4 == 0 && p.n >= 64;
+    if (direct && p.n == 64 && kr < kB3NarrowK) return tiles > 256 && tiles <= 512;
+    return kr >= kB3LoneK + (direct ? 1 : 0) || tiles > 256;
 }
 
 // The block tile: the least estimated time.  A block takes `fixed` us (first stage, check, stores) and per step of 16 k

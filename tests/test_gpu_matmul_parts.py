@@ -35,7 +35,7 @@ def check(a, b, got=None):
 
 # Every form of the kernel: the tiles with whole pairs of steps (128x128, 128x64, 64x64 several per CU, 64x64 with loading
 # waves), K tails in 16-byte loads (128x128 and 64x64) and in scalar ones (both), the ranges of a split product
-FORMS = [(4096, 256, 1024), (1100, 384, 960), (4096, 256, 1152), (1024, 512, 512), (1536, 516, 1600), (600, 516, 516),
+FORMS = [(4096, 256, 1024), (1100, 384, 960), (4096, 256, 1152), (1024, 576, 512), (1536, 516, 1600), (600, 516, 516),
          (1500, 533, 1601), (256, 533, 70), (640, 3072, 640)]
 # and edges in both directions, single rows and few columns, the first K with a CU per tile
 SHAPES = FORMS + [(4096, 384, 384), (1000, 320, 4100), (788, 768, 768), (129, 516, 65), (2000, 260, 2020), (700, 533, 260),
@@ -142,6 +142,16 @@ def test_short_ranges_of_a_split_product_keep_float32(hip, m, k, n, r):
     assert np.array_equal(got[:8, cols], ref)
 
 
+@pytest.mark.parametrize("b,m,k,n", [(96, 512, 512, 64), (96, 100, 640, 64), (4, 512, 512, 512)])
+def test_narrow_and_lone_products_keep_float32(hip, b, m, k, n):
+    """64 columns with K below 1024, and K up to 512 with a CU per tile, run on the fp32 MFMA: a float32 chain."""
+    rng = np.random.default_rng(27)
+    a, w = rng.standard_normal((b, m, k)).astype(np.float32), rng.standard_normal((b, k, n)).astype(np.float32)
+    order = np.arange(k).reshape(-1, 2, 8).transpose(0, 2, 1).reshape(-1)
+    got = mm(a, w)
+    assert np.array_equal(got[1, :64], float32_chain(a[1, :64][:, order], w[1][order]))
+
+
 @pytest.mark.parametrize("m,k,n", [(4096, 768, 768), (788, 768, 768), (1100, 384, 1000)])
 def test_parts_time_does_not_depend_on_zeros(hip, m, k, n):
     """Exactly zero results of nonzero rows and columns (integers, sparse operands, a selection) and small values need
@@ -188,10 +198,10 @@ def test_parts_results_do_not_depend_on_the_tile(hip):
 
 
 def test_parts_of_a_long_k_do_not_depend_on_the_tile(hip):
-    """K = 512: 64x64 tiles whole, its parts 128x128, 128x64 and 64x64 with loading waves; rows of subnormals and a few
+    """K = 576: 64x64 tiles whole, its parts 128x128, 128x64 and 64x64 with loading waves; rows of subnormals and a few
     values that are not finite run on the fp32 MFMA in each."""
     rng = np.random.default_rng(12)
-    a, b = rng.standard_normal((4096, 512)).astype(np.float32), rng.standard_normal((512, 1152)).astype(np.float32)
+    a, b = rng.standard_normal((4096, 576)).astype(np.float32), rng.standard_normal((576, 1152)).astype(np.float32)
     a[10] *= np.float32(1e-38)
     a[900, 500], a[70, 3], b[4, 500], b[300, 20] = np.nan, np.inf, np.float32(1e-40), -np.inf
     whole = mm(a, b)
